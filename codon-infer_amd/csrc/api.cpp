@@ -267,7 +267,7 @@ int cih_model_reserve(cih_model *m, int32_t max_batch, int32_t max_seq_len, uint
     if (good && (flags & CIH_OUT_CONTACTS))
         good = ok(dalloc(ws.M, B * n * n, dl)) && ok(dalloc(ws.r, L * H * B * n, dl)) &&
                ok(dalloc(ws.coef, L * H * B, dl)) && ok(dalloc(ws.rowsum, B * H * S, dl)) &&
-               ok(dalloc(ws.colpart, B * H * ((n + 31) / 32) * n, dl));
+               ok(dalloc(ws.colpart, apc_colpart_floats((int)B, (int)H, (int)n), dl));
     if (good && !(flags & CIH_IO_DEVICE)) {
         if (flags & CIH_OUT_LOGITS) good = good && ok(dalloc(ws.o_logits, T * V, dl));
         if (flags & CIH_OUT_HIDDEN) good = good && ok(dalloc(ws.o_hidden, T * d, dl));
@@ -481,7 +481,10 @@ int forward_impl(cih_model *m, const int32_t *tokens, const int32_t *lens, int32
         // probabilities: straight into the attention-map output when exported
         float *P = nullptr;
         int64_t pb = 0, ph = SS;
-        const bool need_P = want_attn || want_contacts || (want_final && l == L - 1);
+        // contacts read the maps of the heads with a nonzero weight only
+        const bool all_P = want_attn || (want_final && l == L - 1);
+        const bool need_P = all_P || (want_contacts && m->nz[l] > 0);
+        const int *order = need_P && !all_P ? m->d_heads + (size_t)l * H : nullptr;
         if (want_attn) {
             P = t_attn + (size_t)l * H * SS;
             pb = (int64_t)L * H * SS;
@@ -527,7 +530,7 @@ int forward_impl(cih_model *m, const int32_t *tokens, const int32_t *lens, int32
                 ProfScope ps(m, CIH_KC_ATTENTION, fl, 16.0 * T * d);
                 float *rsum = want_contacts && m->nz[l] > 0 ? ws.rowsum : nullptr;
                 HIPCHK(launch_attention(ws.qkv, d, H, sm, ws.rope_c, ws.rope_s, ws.ao, af, P, pb, ph, rsum, ws.attp,
-                                        ws.attp_floats, st));
+                                        ws.attp_floats, st, order, m->nz[l]));
             }
             if (want_contacts && m->nz[l] > 0) {
                 ProfScope ps(m, CIH_KC_OTHER, 0, 0);
@@ -595,10 +598,10 @@ int forward_impl(cih_model *m, const int32_t *tokens, const int32_t *lens, int32
             float *rsum = want_contacts && m->nz[l] > 0 ? ws.rowsum : nullptr;
             if (use_img)
                 HIPCHK(launch_attention_img(ws.qkv, d, H, sm, ws.kv_tb, ws.kv_img, ws.rope_c, ws.rope_s, ws.ao, af, P,
-                                            pb, ph, rsum, ws.attp, ws.attp_floats, st));
+                                            pb, ph, rsum, ws.attp, ws.attp_floats, st, order, m->nz[l]));
             else
                 HIPCHK(launch_attention(ws.qkv, d, H, sm, ws.rope_c, ws.rope_s, ws.ao, af, P, pb, ph, rsum, ws.attp,
-                                        ws.attp_floats, st));
+                                        ws.attp_floats, st, order, m->nz[l]));
         }
         if (want_contacts && m->nz[l] > 0) {
             ProfScope ps(m, CIH_KC_OTHER, 0, 0);
@@ -630,7 +633,8 @@ int forward_impl(cih_model *m, const int32_t *tokens, const int32_t *lens, int32
     }
     if (want_contacts) {
         ProfScope ps(m, CIH_KC_OTHER, 0, 0);
-        HIPCHK(launch_apc_finalize(ws.M, ws.r, ws.coef, m->d_contact_w, L * H, sm, m->contact_b, t_contacts, n_max, st));
+        HIPCHK(launch_apc_finalize(ws.M, ws.r, ws.coef, m->d_contact_w, m->d_lhs, m->n_lhs, sm, m->contact_b,
+                                   t_contacts, n_max, st));
     }
     // final LayerNorm: state.x = LN_f(x) (lib.rs:5379-5387).  It also
     // reports a residual row that is no longer finite (the f16 limbs hold

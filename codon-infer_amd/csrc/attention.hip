@@ -48,6 +48,11 @@
 
 namespace cih {
 
+// What a kernel does with the probabilities of its heads: nothing (one-pass
+// softmax), stores every head's, or stores those of the head slots below
+// nexp only (contacts read the heads with a nonzero weight alone).
+enum { ATT_EXPORT = 0, ATT_ONEPASS = 1, ATT_MIXED = 2 };
+
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
@@ -420,7 +425,8 @@ __global__ __launch_bounds__(NTH, ONEPASS || HD <= 32 ? 4 : 2) void k_attention_
                                                      void *__restrict__ out, int out_fmt, float *__restrict__ P,
                                                      long long pb, long long ph, float inv_scale,
                                                      float *__restrict__ rowsum, int H, int nq, int nfull, int nsplit,
-                                                     float *__restrict__ part) {
+                                                     float *__restrict__ part, const int *__restrict__ order,
+                                                     int nexp) {
     // no FMA contraction: the staged and the image kernel round alike
 #pragma clang fp contract(off)
     constexpr int HALF = HD / 2;
@@ -443,7 +449,9 @@ __global__ __launch_bounds__(NTH, ONEPASS || HD <= 32 ? 4 : 2) void k_attention_
         ks = t % nsplit;
         ns = nsplit;
     }
-    const int qb = task % nq, h = (task / nq) % H, b = task / nq / H;
+    // head slot: the order of heads, exported ones first (null: all in order)
+    const int qb = task % nq, slot = (task / nq) % H, b = task / nq / H;
+    const int h = order ? order[slot] : slot;
     const int len = lens[b], base = cu[b];
     const int qblk = qb * (NTH / 2);  // 32 queries per wave
     if (qblk >= len) return;
@@ -742,7 +750,8 @@ __global__ __launch_bounds__(NTH, ONEPASS || HD <= 32 ? 4 : 2) void k_attention_
         const float mx = fmaxf(m, mo);
         const float inv_sum = 1.0f / (l * __builtin_amdgcn_exp2f(m - mx) + lo * __builtin_amdgcn_exp2f(mo - mx));
         // pass 2: normalized probabilities, optional export, P.V
-        float *Prow = (P && qi < len) ? P + b * pb + h * ph + (size_t)qi * S_max : nullptr;
+        const bool exported = slot < nexp;
+        float *Prow = (P && exported && qi < len) ? P + b * pb + h * ph + (size_t)qi * S_max : nullptr;
         float rs = 0.0f;  // sum of this query's probabilities over residue keys (contacts)
         sweep(true, [&](int kt0) __attribute__((always_inline)) {
             f32x16 acc;
@@ -754,10 +763,10 @@ __global__ __launch_bounds__(NTH, ONEPASS || HD <= 32 ? 4 : 2) void k_attention_
                 p[q] = key < len ? __builtin_amdgcn_exp2f(acc[q] - mx) * inv_sum : 0.0f;
             }
             if (Prow) store_p(Prow, p, kt0 + 4 * hh, len);
-            if (rowsum) rs += tile_residue_sum(p, kt0, hh, len);
+            if (rowsum && exported) rs += tile_residue_sum(p, kt0, hh, len);
             pv(oacc, p);
         });
-        write_rowsum(rowsum, rs, b, h, H, S_max, qi, len, hh);
+        write_rowsum(exported ? rowsum : nullptr, rs, b, h, H, S_max, qi, len, hh);
         out_scale = 1.0f;
     }
     if (qi < len) {
@@ -786,24 +795,26 @@ __global__ __launch_bounds__(NTH, ONEPASS || HD <= 32 ? 4 : 2) void k_attention_
 // 32-key tiles w, w + KS, ...  Each wave stages its tiles (RoPE, limbs, V
 // transposed, as k_attention_h stages them) in its own LDS, so the waves
 // meet only to combine:
-//  * with the export (ONEPASS false): pass 1's running maxima and sums (per
+//  * with the export: pass 1's running maxima and sums (per
 //    wave and lane) give each query's maximum M and sum L = sum 2^(m_s - M)
 //    l_s in wave order; pass 2 stores the probabilities exp2(s - M) / L and
 //    the waves' P.V accumulators are added in wave order;
-//  * without (ONEPASS): each wave runs the one-pass online softmax over its
+//  * without: each wave runs the one-pass online softmax over its
 //    tiles (online_tile, as k_attention_h), and the waves' results combine
 //    as key ranges do in k_attention_merge: O = sum 2^(m_s - M) o_s /
 //    sum 2^(m_s - M) l_s, in wave order.
 // Per query the arithmetic is k_attention_h's, with the softmax and P.V sums
 // regrouped by wave: agreement to rounding, not bit for bit.
-template <int HD, int KS, bool ONEPASS>
+// MODE: ATT_ONEPASS, ATT_EXPORT, or ATT_MIXED (head slots below nexp export).
+template <int HD, int KS, int MODE>
 __global__ __launch_bounds__(64 * KS) void k_attention_xs(const float *__restrict__ qkv, int d,
                                                           const int *__restrict__ cu, const int *__restrict__ lens,
                                                           int S_max, const float *__restrict__ rc,
                                                           const float *__restrict__ rsn, void *__restrict__ out,
                                                           int out_fmt, float *__restrict__ P, long long pb,
                                                           long long ph, float inv_scale, float *__restrict__ rowsum,
-                                                          int H, int nq) {
+                                                          int H, int nq, const int *__restrict__ order,
+                                                          int nexp) {
 #pragma clang fp contract(off)
     constexpr int HALF = HD / 2;
     constexpr int HDP = (HD + 15) / 16 * 16;
@@ -819,7 +830,8 @@ __global__ __launch_bounds__(64 * KS) void k_attention_xs(const float *__restric
     __shared__ float red[KS][3][64];  // per wave and lane: running max, sum, residue sum
     static_assert((STAGE_BYTES > OX_BYTES ? STAGE_BYTES : OX_BYTES) + KS * 3 * 64 * 4 <= 160 * 1024, "LDS");
 
-    const int task = blockIdx.x, qb = task % nq, h = (task / nq) % H, b = task / nq / H;
+    const int task = blockIdx.x, qb = task % nq, slot = (task / nq) % H, b = task / nq / H;
+    const int h = order ? order[slot] : slot;
     const int len = lens[b], base = cu[b];
     const int qblk = qb * 32;
     if (qblk >= len) return;
@@ -985,7 +997,8 @@ __global__ __launch_bounds__(64 * KS) void k_attention_xs(const float *__restric
                     v;
         }
     };
-    if constexpr (ONEPASS) {
+    // a head without an export (uniform over the workgroup)
+    if (MODE == ATT_ONEPASS || (MODE == ATT_MIXED && slot >= nexp)) {
         f32x16 oacc[DT];
 #pragma unroll
         for (int t = 0; t < DT; t++)
@@ -1027,7 +1040,8 @@ __global__ __launch_bounds__(64 * KS) void k_attention_xs(const float *__restric
         __syncthreads();
         if (w == 0) finish(1.0f / L);
         return;
-    } else {
+    }
+    if constexpr (MODE != ATT_ONEPASS) {
         // pass 1: running max / sum of exp per lane over this wave's tiles
         float m = -INFINITY, l = 0.0f;
         for (int t = w; t < ntile; t += KS) {
@@ -1173,13 +1187,21 @@ __device__ __forceinline__ void dma16(const void *g, unsigned lds_base) {
 // a score exceeds it by more than 8 (base-2 units), so the accumulators are
 // rescaled rarely and p <= 256 (the normalisation is unchanged: o / l with o
 // and l under the same offset).
-template <int HD, bool ONEPASS, int NTH>
-__global__ __launch_bounds__(NTH, ONEPASS || HD <= 32 ? 4 : 2) void k_attention_img(
+//
+// MODE: ATT_ONEPASS, ATT_EXPORT (two passes, P stored), or ATT_MIXED: head
+// slots below nexp export, the others take the one-pass softmax.  The mixed
+// grid runs slot by slot over the batch, so the two-pass heads start first.
+// ESM-2's contact heads weight 17-38% of the heads, and a two-pass head costs
+// about twice a one-pass one plus its stores: 150M Q4_0 B=4 L=1024 with
+// contacts 10.72 -> 7.07 ms per forward, together with the contact kernels
+// reading those heads only (650M Q8_0 L=257: 4.33 -> 3.47 ms).
+template <int HD, int MODE, int NTH>
+__global__ __launch_bounds__(NTH, MODE != ATT_EXPORT || HD <= 32 ? 4 : 2) void k_attention_img(
     const float *__restrict__ qkv, int d, const int *__restrict__ cu, const int *__restrict__ lens, int S_max,
     const int *__restrict__ tb, const unsigned char *__restrict__ img, const float *__restrict__ rc,
     const float *__restrict__ rsn, void *__restrict__ out, int out_fmt, float *__restrict__ P, long long pb,
     long long ph, float inv_scale, float *__restrict__ rowsum, int H, int nq, int nfull, int nsplit,
-    float *__restrict__ part, int xcd_pairs) {
+    float *__restrict__ part, int xcd_pairs, const int *__restrict__ order, int nexp, int nb) {
     // no FMA contraction: the staged and the image kernel round alike
 #pragma clang fp contract(off)
     using I = KvImg<HD>;
@@ -1203,7 +1225,9 @@ __global__ __launch_bounds__(NTH, ONEPASS || HD <= 32 ? 4 : 2) void k_attention_
         const int g = task / (8 * nq), r = task % (8 * nq);
         task = (8 * g + r % 8) * nq + r / 8;
     }
-    const int qb = task % nq, h = (task / nq) % H, b = task / nq / H;
+    const int qb = task % nq, slot = MODE == ATT_MIXED ? task / nq / nb : (task / nq) % H;
+    const int b = MODE == ATT_MIXED ? (task / nq) % nb : task / nq / H;
+    const int h = MODE == ATT_MIXED ? order[slot] : slot;
     const int len = lens[b], base = cu[b];
     const int qblk = qb * (NTH / 2);
     if (qblk >= len) return;
@@ -1309,7 +1333,7 @@ __global__ __launch_bounds__(NTH, ONEPASS || HD <= 32 ? 4 : 2) void k_attention_
 #pragma unroll
         for (int q = 0; q < 16; q++) oacc[t][q] = 0.0f;
     float out_scale;
-    if constexpr (ONEPASS) {
+    if (MODE == ATT_ONEPASS || (MODE == ATT_MIXED && slot >= nexp)) {
         float m = -INFINITY, l = 0.0f;
         sweep(std::true_type{}, [&](const unsigned char *st, int kt0, auto masked) __attribute__((always_inline)) {
             online_tile<DT, decltype(masked)::value>(
@@ -1335,7 +1359,7 @@ __global__ __launch_bounds__(NTH, ONEPASS || HD <= 32 ? 4 : 2) void k_attention_
             return;
         }
         out_scale = 1.0f / lt;
-    } else {
+    } else if constexpr (MODE != ATT_ONEPASS) {
         // pass 1 (K limbs only): running max / sum of exp per lane
         float m = -INFINITY, l = 0.0f;
         sweep(std::false_type{}, [&](const unsigned char *st, int kt0, auto masked) __attribute__((always_inline)) {
@@ -1536,10 +1560,12 @@ size_t attention_part_floats(int hd) { return (size_t)device_cus() * 512 * (hd +
 
 hipError_t launch_attention(const float *qkv, int d, int H, SeqMeta sm, const float *rope_cos, const float *rope_sin,
                             void *out, int out_fmt, float *P, int64_t pb, int64_t ph, float *rowsum, float *part,
-                            size_t part_floats, hipStream_t st) {
+                            size_t part_floats, hipStream_t st, const int *order, int nexp) {
     if (rowsum && !P) return hipErrorInvalidValue;
     if ((out_fmt == AF_X3 || out_fmt == AF_H2) && d % 32) return hipErrorInvalidValue;
     const int hd = d / H;
+    if (!order) nexp = H;
+    const bool mixed = P && nexp < H;
     const float inv_scale = 1.0f / sqrtf((float)hd);
     const char *e = getenv("CIH_ATT");
     const bool fp32 = (e && !strcmp(e, "fp32")) || full_range_mode();
@@ -1599,16 +1625,15 @@ hipError_t launch_attention(const float *qkv, int d, int H, SeqMeta sm, const fl
 #define CIH_ATT_H(HDV, ONE, NTH)                                                                                 \
     hipLaunchKernelGGL((k_attention_h<HDV, ONE, NTH>), dim3(grid), dim3(NTH), 0, st, qkv, d, sm.cu, sm.lens,     \
                        sm.S_max, rope_cos, rope_sin, out, out_fmt, P, (long long)pb, (long long)ph, inv_scale, rowsum, \
-                       H, nq, nfull, nsplit, part)
+                       H, nq, nfull, nsplit, part, order, nexp)
+#define CIH_ATT_XS(HDV, MODE)                                                                                   \
+    hipLaunchKernelGGL((k_attention_xs<HDV, 8, MODE>), dim3(t32), dim3(512), 0, st, qkv, d, sm.cu, sm.lens,      \
+                       sm.S_max, rope_cos, rope_sin, out, out_fmt, P, (long long)pb, (long long)ph, inv_scale,   \
+                       rowsum, H, nq32, order, nexp)
 #define CIH_ATT(HDV)                                                                                           \
-    if (xsplit && P)                                                                                            \
-        hipLaunchKernelGGL((k_attention_xs<HDV, 8, false>), dim3(t32), dim3(512), 0, st, qkv, d, sm.cu, sm.lens, \
-                           sm.S_max, rope_cos, rope_sin, out, out_fmt, P, (long long)pb, (long long)ph, inv_scale, \
-                           rowsum, H, nq32);                                                                    \
-    else if (xsplit)                                                                                            \
-        hipLaunchKernelGGL((k_attention_xs<HDV, 8, true>), dim3(t32), dim3(512), 0, st, qkv, d, sm.cu, sm.lens,  \
-                           sm.S_max, rope_cos, rope_sin, out, out_fmt, P, (long long)pb, (long long)ph, inv_scale, \
-                           rowsum, H, nq32);                                                                    \
+    if (xsplit && mixed) CIH_ATT_XS(HDV, ATT_MIXED);                                                            \
+    else if (xsplit && P) CIH_ATT_XS(HDV, ATT_EXPORT);                                                          \
+    else if (xsplit) CIH_ATT_XS(HDV, ATT_ONEPASS);                                                              \
     else if (fp32 && P) CIH_ATT_K(k_attention, HDV, false);                                                     \
     else if (fp32) CIH_ATT_K(k_attention, HDV, true);                                                           \
     else if (P && wide) CIH_ATT_H(HDV, false, 512);                                                             \
@@ -1631,6 +1656,7 @@ hipError_t launch_attention(const float *qkv, int d, int H, SeqMeta sm, const fl
     }
 #undef CIH_ATT
 #undef CIH_ATT_H
+#undef CIH_ATT_XS
 #undef CIH_ATT_K
     return hipGetLastError();
 }
@@ -1688,11 +1714,14 @@ hipError_t launch_kv_prep(const float *qkv, int d, int H, const int *ti, int til
 
 hipError_t launch_attention_img(const float *qkv, int d, int H, SeqMeta sm, const int *tb, const unsigned char *img,
                                 const float *rope_cos, const float *rope_sin, void *out, int out_fmt, float *P,
-                                int64_t pb, int64_t ph, float *rowsum, float *part, size_t part_floats, hipStream_t st) {
+                                int64_t pb, int64_t ph, float *rowsum, float *part, size_t part_floats, hipStream_t st,
+                                const int *order, int nexp) {
     if (rowsum && !P) return hipErrorInvalidValue;
     if ((out_fmt == AF_X3 || out_fmt == AF_H2) && d % 32) return hipErrorInvalidValue;
     const int hd = d / H;
     if (!attention_img_supported(hd) || d != hd * H) return hipErrorInvalidValue;
+    if (!order) nexp = H;
+    const bool mixed = P && nexp < H;
     const float inv_scale = 1.0f / sqrtf((float)hd);
     // query blocks and key split as in launch_attention
     const char *qe = getenv("CIH_ATT_QB");
@@ -1720,12 +1749,14 @@ hipError_t launch_attention_img(const float *qkv, int d, int H, SeqMeta sm, cons
 #define CIH_ATI(HDV, ONE, NTH)                                                                                   \
     hipLaunchKernelGGL((k_attention_img<HDV, ONE, NTH>), dim3(grid), dim3(NTH), 0, st, qkv, d, sm.cu, sm.lens,    \
                        sm.S_max, tb, img, rope_cos, rope_sin, out, out_fmt, P, (long long)pb, (long long)ph,      \
-                       inv_scale, rowsum, H, nq, nfull, nsplit, part, xcd_pairs)
+                       inv_scale, rowsum, H, nq, nfull, nsplit, part, xcd_pairs, order, nexp, sm.B)
 #define CIH_ATI_HD(HDV)                                                                                          \
-    if (P && wide) CIH_ATI(HDV, false, 512);                                                                      \
-    else if (P) CIH_ATI(HDV, false, 256);                                                                         \
-    else if (wide) CIH_ATI(HDV, true, 512);                                                                       \
-    else CIH_ATI(HDV, true, 256);                                                                                 \
+    if (mixed && wide) CIH_ATI(HDV, ATT_MIXED, 512);                                                              \
+    else if (mixed) CIH_ATI(HDV, ATT_MIXED, 256);                                                                 \
+    else if (P && wide) CIH_ATI(HDV, ATT_EXPORT, 512);                                                            \
+    else if (P) CIH_ATI(HDV, ATT_EXPORT, 256);                                                                    \
+    else if (wide) CIH_ATI(HDV, ATT_ONEPASS, 512);                                                                \
+    else CIH_ATI(HDV, ATT_ONEPASS, 256);                                                                                 \
     if (nsplit > 1) {                                                                                             \
         const long n = (long)(tasks - nfull) * QB * (HDV / 4);                                                    \
         hipLaunchKernelGGL((k_attention_merge<HDV>), dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, part,   \

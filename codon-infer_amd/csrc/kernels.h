@@ -361,14 +361,17 @@ hipError_t launch_layernorm(const float *x, const float *w, const float *b, void
 // Bidirectional rotary attention over packed Q|K|V rows.  When P != nullptr
 // every softmax row is stored at P[b*pb + h*ph + q*S_max + k]; rowsum (with
 // P) receives rowsum[b][h][q] = sum of row q over the residue keys 1..len-2,
-// for residue queries.
+// for residue queries.  order (with P): a device list of all H heads, of
+// which the first nexp are exported (P and rowsum) and the others only
+// attended (nullptr: every head is exported).
 // out: [T][d] FP32 (out_fmt AF_F32) or a limb format (AF_X3 / AF_H2).
 // Without P, tasks that would leave workgroup slots idle are split over key
 // ranges whose partial results (part, part_floats floats; nullptr: no split)
 // a merge kernel combines; attention_part_floats(hd) floats always suffice.
 hipError_t launch_attention(const float *qkv, int d, int H, SeqMeta sm, const float *rope_cos,
                             const float *rope_sin, void *out, int out_fmt, float *P, int64_t pb, int64_t ph,
-                            float *rowsum, float *part, size_t part_floats, hipStream_t st);
+                            float *rowsum, float *part, size_t part_floats, hipStream_t st,
+                            const int *order = nullptr, int nexp = 0);
 size_t attention_part_floats(int hd);
 
 // The same attention with K and V taken from the tile images of kv_image.h
@@ -376,7 +379,8 @@ size_t attention_part_floats(int hd);
 // first tile row of each sequence.  hd 16, 32 or 64.
 hipError_t launch_attention_img(const float *qkv, int d, int H, SeqMeta sm, const int *tb, const unsigned char *img,
                                 const float *rope_cos, const float *rope_sin, void *out, int out_fmt, float *P,
-                                int64_t pb, int64_t ph, float *rowsum, float *part, size_t part_floats, hipStream_t st);
+                                int64_t pb, int64_t ph, float *rowsum, float *part, size_t part_floats, hipStream_t st,
+                                const int *order = nullptr, int nexp = 0);
 
 // Per-forward set-up of the tile images: tb[b] = first tile row of sequence
 // b, pk / pos of every packed token, ti[tile row] = (first packed row, keys,
@@ -404,14 +408,17 @@ hipError_t launch_head_mean(const float *P, int64_t pb, int64_t ph, int H, SeqMe
 // Contacts (APC).  For layer l, heads with w != 0, one read of the maps:
 //   M[b][i][j] += sum_h w_lh * P_lh[i+1][j+1]
 //   r[l][h][b][i] = rowsum[b][h][i+1] + sum_j P_lh[j+1][i+1]   (residues only)
-// rowsum comes from launch_attention; colpart: [B][H][ceil(n_max/32)][n_max] scratch.
+// rowsum comes from launch_attention; colpart: scratch of
+// apc_colpart_floats(B, H, n_max) floats.
+size_t apc_colpart_floats(int B, int H, int n_max);
 hipError_t launch_apc_layer(const float *P, int64_t pb, int64_t ph, int H, int l, const float *w_dev,
                             const int *heads_dev, int n_heads_nz, SeqMeta sm, const float *rowsum, float *colpart,
                             float *M, float *r, hipStream_t st);
 // contacts[b][i][j] = sigmoid(M_ij + M_ji - sum_lh (w_lh / T_lh) r_i r_j + bias)
-// coef: [L*H][B] scratch for w_lh / T_lh.
-hipError_t launch_apc_finalize(const float *M, const float *r, float *coef, const float *w_dev, int LH, SeqMeta sm,
-                               float bias, float *contacts, int n_stride, hipStream_t st);
+// over the nlh layer-heads of nonzero weight, lhs_dev their indices l H + h in
+// order.  coef: [nlh][B] scratch for w_lh / T_lh.
+hipError_t launch_apc_finalize(const float *M, const float *r, float *coef, const float *w_dev, const int *lhs_dev,
+                               int nlh, SeqMeta sm, float bias, float *contacts, int n_stride, hipStream_t st);
 
 // DMS rows (pipeline.rs:152-172): for entry i, logits row meta[2i] of the
 // packed [T][V] logits and wild-type token meta[2i+1] give out[i][0..19] =

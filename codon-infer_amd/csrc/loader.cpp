@@ -494,12 +494,21 @@ int create(const cih_config &cfg, const Layout &y, int dst_dt, int fd, const std
     m->nz.assign(L, 0);
     if (m->has_contacts) {
         m->contact_w.assign(contact_w, contact_w + L * H);
-        std::vector<int> heads(L * H, 0);
-        for (int64_t l = 0; l < L; l++)
+        std::vector<int> heads(L * H, 0), lhs;
+        for (int64_t l = 0; l < L; l++) {
             for (int64_t h = 0; h < H; h++)
-                if (m->contact_w[l * H + h] != 0.0f) heads[l * H + m->nz[l]++] = (int)h;
+                if (m->contact_w[l * H + h] != 0.0f) {
+                    heads[l * H + m->nz[l]++] = (int)h;
+                    lhs.push_back((int)(l * H + h));
+                }
+            int at = m->nz[l];
+            for (int64_t h = 0; h < H; h++)
+                if (!(m->contact_w[l * H + h] != 0.0f)) heads[l * H + at++] = (int)h;
+        }
+        m->n_lhs = (int)lhs.size();
         int rc = upload(m, m->d_contact_w, m->contact_w.data(), m->contact_w.size());
         if (!rc) rc = upload(m, m->d_heads, heads.data(), heads.size());
+        if (!rc) rc = upload(m, m->d_lhs, lhs.data(), lhs.size());
         if (rc) return fail(rc);
     }
     *out = m;

@@ -1,5 +1,7 @@
 // Memory-bound kernels of the forward: embedding, LayerNorm, last-layer head
 // mean, contact-map (APC) statistics and finalisation, output scatter.
+#include <algorithm>
+
 #include "kernels.h"
 
 namespace cih {
@@ -274,25 +276,46 @@ hipError_t launch_head_mean(const float *P, int64_t pb, int64_t ph, int H, SeqMe
 // Summed over heads: logit = M + M^T - sum_h (w_h / T_h) r_h r_h^T with
 // M = sum_h w_h A_h, and r_i = (row sum of A)_i + (column sum of A)_i.  The
 // attention kernel supplies the row sums; k_apc_tile reads each map once,
-// accumulating M and per-32-row column partial sums, which k_apc_r adds in
-// order.  M: [B][n_max][n_max], r: [L*H][B][n_max], n_max = S_max - 2.
-constexpr int APC_ROWS = 32;  // map rows per workgroup of k_apc_tile
-constexpr int APC_HMAX = 40;  // most heads of any preset (3B)
+// accumulating M and column partial sums of `rows` map rows, which k_apc_r
+// adds in order.  M: [B][n_max][n_max], r: [L*H][B][n_max], n_max = S_max - 2.
+constexpr int APC_HMAX = 40;     // most heads of any preset (3B)
+constexpr int APC_ROWS_MIN = 8;  // map rows per wave of k_apc_tile: 8, 16 or 32
 
-// HM >= nz heads per pass with branch-free loads (heads past nz repeat head
-// nz - 1 with weight 0 and are not written), two map rows per step, so a
-// thread has 2 * HM loads in flight.
-template <int HM>
-__global__ __launch_bounds__(256) void k_apc_tile(const float *__restrict__ P, long long pb, long long ph, int H,
-                                                  int l, const float *__restrict__ w, const int *__restrict__ heads,
-                                                  int nz, const int *__restrict__ lens, int S_max,
-                                                  float *__restrict__ M, float *__restrict__ colpart, int B) {
+// Map rows per wave: 32, fewer where that leaves the device short of the
+// eight waves per CU that keep enough loads in flight (one 255-residue
+// protein: 8 tiles of 32 rows x 4 column groups).  More tiles mean more
+// partial sums for k_apc_r.
+static int apc_rows(int B, int n_max) {
+    int rows = 32;
+    while (rows > APC_ROWS_MIN && (long)B * ((n_max + rows - 1) / rows) * ((n_max + 63) / 64) < 8L * device_cus())
+        rows /= 2;
+    return rows;
+}
+
+// Enough for every call of at most B sequences and n_max residues: whole
+// 32-row tiles, or, where the rows were halved, fewer than 2 x 8 waves per CU
+// of 64 columns each.
+size_t apc_colpart_floats(int B, int H, int n_max) {
+    return (size_t)H * std::max((size_t)B * ((n_max + 31) / 32) * n_max, (size_t)2 * 8 * device_cus() * 64);
+}
+
+// One wave = 64 residue columns x `rows` map rows.  HM >= nz heads per pass
+// with branch-free loads (heads past nz repeat head nz - 1 with weight 0 and
+// are not written), R map rows per step, so a lane has R * HM loads in flight.
+// Bound by the maps' bytes (nz n^2 floats) and the accumulator's (twice n^2);
+// the launch takes the smallest HM that holds the layer's heads, so that no
+// map is read for nothing.
+template <int HM, int R>
+__global__ __launch_bounds__(64) void k_apc_tile(const float *__restrict__ P, long long pb, long long ph, int H,
+                                                 int l, const float *__restrict__ w, const int *__restrict__ heads,
+                                                 int nz, const int *__restrict__ lens, int S_max, int rows,
+                                                 float *__restrict__ M, float *__restrict__ colpart, int B) {
     const int tile = blockIdx.x, b = blockIdx.z;
-    const int n = lens[b] - 2, n_max = S_max - 2, ntiles = (n_max + APC_ROWS - 1) / APC_ROWS;
-    const int j = blockIdx.y * 256 + threadIdx.x;  // residue column
-    const int i0 = tile * APC_ROWS;
+    const int n = lens[b] - 2, n_max = S_max - 2, ntiles = (n_max + rows - 1) / rows;
+    const int j = blockIdx.y * 64 + threadIdx.x;  // residue column
+    const int i0 = tile * rows;
     if (j >= n || i0 >= n) return;
-    const int i1 = min(i0 + APC_ROWS, n);
+    const int i1 = min(i0 + rows, n);
     long long off[HM];
     float wk[HM], cs[HM];
 #pragma unroll
@@ -305,56 +328,68 @@ __global__ __launch_bounds__(256) void k_apc_tile(const float *__restrict__ P, l
     const float *P0 = P + b * pb + S_max + 1 + j;  // row i + 1, column j + 1
     float *M0 = M + (size_t)b * n_max * n_max + j;
     int i = i0;
-    for (; i + 2 <= i1; i += 2) {
-        const float *r0 = P0 + (size_t)i * S_max, *r1 = r0 + S_max;
-        float a0[HM], a1[HM];
+    for (; i + R <= i1; i += R) {
+        float a[R][HM], acc[R];
 #pragma unroll
-        for (int k = 0; k < HM; k++) {
-            a0[k] = r0[off[k]];
-            a1[k] = r1[off[k]];
-        }
-        float acc0 = M0[(size_t)i * n_max], acc1 = M0[(size_t)(i + 1) * n_max];
+        for (int r = 0; r < R; r++) {
+            const float *row = P0 + (size_t)(i + r) * S_max;
 #pragma unroll
-        for (int k = 0; k < HM; k++) {
-            acc0 += wk[k] * a0[k];
-            cs[k] += a0[k];
+            for (int k = 0; k < HM; k++) a[r][k] = row[off[k]];
+            acc[r] = M0[(size_t)(i + r) * n_max];
         }
 #pragma unroll
-        for (int k = 0; k < HM; k++) {
-            acc1 += wk[k] * a1[k];
-            cs[k] += a1[k];
+        for (int r = 0; r < R; r++) {
+#pragma unroll
+            for (int k = 0; k < HM; k++) {
+                acc[r] += wk[k] * a[r][k];
+                cs[k] += a[r][k];
+            }
+            M0[(size_t)(i + r) * n_max] = acc[r];
         }
-        M0[(size_t)i * n_max] = acc0;
-        M0[(size_t)(i + 1) * n_max] = acc1;
     }
-    if (i < i1) {
-        const float *r0 = P0 + (size_t)i * S_max;
-        float acc0 = M0[(size_t)i * n_max];
+    for (; i < i1; i++) {
+        const float *row = P0 + (size_t)i * S_max;
+        float acc = M0[(size_t)i * n_max];
 #pragma unroll
         for (int k = 0; k < HM; k++) {
-            const float a = r0[off[k]];
-            acc0 += wk[k] * a;
+            const float a = row[off[k]];
+            acc += wk[k] * a;
             cs[k] += a;
         }
-        M0[(size_t)i * n_max] = acc0;
+        M0[(size_t)i * n_max] = acc;
     }
 #pragma unroll
     for (int k = 0; k < HM; k++)
-        if (k < nz) colpart[(((size_t)b * H + heads[k]) * ntiles + tile) * n_max + j] = cs[k];
+        if (k < nz) colpart[(((size_t)b * nz + k) * ntiles + tile) * n_max + j] = cs[k];
 }
 
-// r[l*H + h][b][i] = rowsum[b][h][i+1] + column partials of i in tile order
+// r[l*H + h][b][i] = rowsum[b][h][i+1] + column partials of i in tile order,
+// four waves of every fourth group of 8 tiles (8 loads in flight each) joined
+// in wave order
 __global__ __launch_bounds__(256) void k_apc_r(const float *__restrict__ rowsum, const float *__restrict__ colpart,
-                                               int H, int l, const int *__restrict__ heads,
-                                               const int *__restrict__ lens, int S_max, float *__restrict__ r,
-                                               int B) {
-    const int b = blockIdx.z, h = heads[blockIdx.y];
-    const int n = lens[b] - 2, n_max = S_max - 2, ntiles = (n_max + APC_ROWS - 1) / APC_ROWS;
-    const int i = blockIdx.x * 256 + threadIdx.x;
-    if (i >= n) return;
+                                               int H, int l, const int *__restrict__ heads, int nz,
+                                               const int *__restrict__ lens, int S_max, int rows,
+                                               float *__restrict__ r, int B) {
+    const int b = blockIdx.z, k = blockIdx.y, h = heads[k];
+    const int n = lens[b] - 2, n_max = S_max - 2, ntiles = (n_max + rows - 1) / rows;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, i = blockIdx.x * 64 + lane;
+    __shared__ float part[3][64];
+    const int nt = n > 0 ? (n + rows - 1) / rows : 0;
+    const float *cp = colpart + ((size_t)b * nz + k) * ntiles * n_max + i;
     float c = 0.0f;
-    const int nt = (n + APC_ROWS - 1) / APC_ROWS;
-    for (int t = 0; t < nt; t++) c += colpart[(((size_t)b * H + h) * ntiles + t) * n_max + i];
+    if (i < n)
+        for (int t0 = wave * 8; t0 < nt; t0 += 32) {
+            float v[8];
+#pragma unroll
+            for (int e = 0; e < 8; e++) v[e] = cp[(size_t)min(t0 + e, nt - 1) * n_max];
+#pragma unroll
+            for (int e = 0; e < 8; e++)
+                if (t0 + e < nt) c += v[e];
+        }
+    if (wave) part[wave - 1][lane] = c;
+    __syncthreads();
+    if (wave || i >= n) return;
+    c = ((c + part[0][lane]) + part[1][lane]) + part[2][lane];
     r[((size_t)(l * H + h) * B + b) * n_max + i] = rowsum[((size_t)b * H + h) * S_max + i + 1] + c;
 }
 
@@ -363,35 +398,38 @@ hipError_t launch_apc_layer(const float *P, int64_t pb, int64_t ph, int H, int l
                             float *M, float *r, hipStream_t st) {
     if (n_heads_nz <= 0 || sm.S_max < 3) return hipSuccess;
     if (n_heads_nz > APC_HMAX || H > APC_HMAX) return hipErrorInvalidValue;
-    const int n_max = sm.S_max - 2;
-    const dim3 tg((n_max + APC_ROWS - 1) / APC_ROWS, (n_max + 255) / 256, sm.B);
-    if (n_heads_nz <= 20)
-        hipLaunchKernelGGL(k_apc_tile<20>, tg, dim3(256), 0, st, P, (long long)pb, (long long)ph, H, l, w_dev, heads_dev,
-                           n_heads_nz, sm.lens, sm.S_max, M, colpart, sm.B);
-    else
-        hipLaunchKernelGGL(k_apc_tile<APC_HMAX>, tg, dim3(256), 0, st, P, (long long)pb, (long long)ph, H, l, w_dev,
-                           heads_dev, n_heads_nz, sm.lens, sm.S_max, M, colpart, sm.B);
-    hipLaunchKernelGGL(k_apc_r, dim3((n_max + 255) / 256, n_heads_nz, sm.B), dim3(256), 0, st, rowsum, colpart, H, l,
-                       heads_dev, sm.lens, sm.S_max, r, sm.B);
+    const int n_max = sm.S_max - 2, rows = apc_rows(sm.B, n_max);
+    const dim3 tg((n_max + rows - 1) / rows, (n_max + 63) / 64, sm.B);
+#define CIH_APC(HM, R)                                                                                              \
+    hipLaunchKernelGGL((k_apc_tile<HM, R>), tg, dim3(64), 0, st, P, (long long)pb, (long long)ph, H, l, w_dev,       \
+                       heads_dev, n_heads_nz, sm.lens, sm.S_max, rows, M, colpart, sm.B)
+    if (n_heads_nz <= 2) CIH_APC(2, 8);
+    else if (n_heads_nz <= 4) CIH_APC(4, 8);
+    else if (n_heads_nz <= 7) CIH_APC(7, 4);
+    else if (n_heads_nz <= 12) CIH_APC(12, 4);
+    else if (n_heads_nz <= 20) CIH_APC(20, 2);
+    else CIH_APC(APC_HMAX, 2);
+#undef CIH_APC
+    hipLaunchKernelGGL(k_apc_r, dim3((n_max + 63) / 64, n_heads_nz, sm.B), dim3(256), 0, st, rowsum, colpart, H, l,
+                       heads_dev, n_heads_nz, sm.lens, sm.S_max, rows, r, sm.B);
     return hipGetLastError();
 }
 
-// coef[lh][b] = w_lh / T_lh (0 when |T| <= 1e-12 or w == 0), T = sum_i r_i
+// coef[t][b] = w_lh / T_lh of layer-head lh = lhs[t] (0 when |T| <= 1e-12), T = sum_i r_i
 __global__ __launch_bounds__(256) void k_apc_coef(const float *__restrict__ r, const float *__restrict__ w,
-                                                  const int *__restrict__ lens, int S_max, int B,
-                                                  float *__restrict__ coef) {
-    const int lh = blockIdx.x, b = blockIdx.y;
+                                                  const int *__restrict__ lhs, const int *__restrict__ lens, int S_max,
+                                                  int B, float *__restrict__ coef) {
+    const int lh = lhs[blockIdx.x], b = blockIdx.y;
     const int n = lens[b] - 2, n_max = S_max - 2;
     __shared__ float red[4];
     float s = 0.0f;
-    if (w[lh] != 0.0f)
-        for (int i = threadIdx.x; i < n; i += 256) s += r[((size_t)lh * B + b) * n_max + i];
+    for (int i = threadIdx.x; i < n; i += 256) s += r[((size_t)lh * B + b) * n_max + i];
     s = wave_sum(s);
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
     __syncthreads();
     if (threadIdx.x == 0) {
         const float T = red[0] + red[1] + red[2] + red[3];
-        coef[(size_t)lh * B + b] = (w[lh] != 0.0f && fabsf(T) > 1e-12f) ? w[lh] * (1.0f / T) : 0.0f;
+        coef[(size_t)blockIdx.x * B + b] = fabsf(T) > 1e-12f ? w[lh] * (1.0f / T) : 0.0f;
     }
 }
 
@@ -402,9 +440,9 @@ __global__ __launch_bounds__(256) void k_apc_coef(const float *__restrict__ r, c
 // form: corr = fma(c, r_i * r_j, corr) in layer-head order, skipping c == 0.
 constexpr int APC_FT = 64, APC_FL = 64;
 __global__ __launch_bounds__(256) void k_apc_final(const float *__restrict__ M, const float *__restrict__ r,
-                                                   const float *__restrict__ coef, int LH, const int *__restrict__ lens,
-                                                   int S_max, int B, float bias, float *__restrict__ out,
-                                                   int n_stride) {
+                                                   const float *__restrict__ coef, const int *__restrict__ lhs,
+                                                   int nlh, const int *__restrict__ lens, int S_max, int B,
+                                                   float bias, float *__restrict__ out, int n_stride) {
     const int b = blockIdx.z, i0 = blockIdx.y * APC_FT, j0 = blockIdx.x * APC_FT;
     const int n = lens[b] - 2, n_max = S_max - 2;
     if (i0 >= n || j0 >= n) return;
@@ -416,18 +454,18 @@ __global__ __launch_bounds__(256) void k_apc_final(const float *__restrict__ M, 
     for (int m = 0; m < 4; m++)
 #pragma unroll
         for (int k = 0; k < 4; k++) corr[m][k] = 0.0f;
-    for (int lh0 = 0; lh0 < LH; lh0 += APC_FL) {
+    for (int lh0 = 0; lh0 < nlh; lh0 += APC_FL) {
         __syncthreads();
         for (int e = tid; e < APC_FL * APC_FT; e += 256) {
-            const int lh = lh0 + e / APC_FT, x = e % APC_FT;
-            const float *rr = r + ((size_t)lh * B + b) * n_max;
-            const bool in = lh < LH;
+            const int t = lh0 + e / APC_FT, x = e % APC_FT;
+            const bool in = t < nlh;
+            const float *rr = r + ((size_t)lhs[in ? t : 0] * B + b) * n_max;
             ri[e / APC_FT][x] = in && i0 + x < n ? rr[i0 + x] : 0.0f;
             rj[e / APC_FT][x] = in && j0 + x < n ? rr[j0 + x] : 0.0f;
         }
-        if (tid < APC_FL) cs[tid] = lh0 + tid < LH ? coef[(size_t)(lh0 + tid) * B + b] : 0.0f;
+        if (tid < APC_FL) cs[tid] = lh0 + tid < nlh ? coef[(size_t)(lh0 + tid) * B + b] : 0.0f;
         __syncthreads();
-        const int nl = min(APC_FL, LH - lh0);
+        const int nl = min(APC_FL, nlh - lh0);
         for (int t = 0; t < nl; t++) {
             const float c = cs[t];
             if (c == 0.0f) continue;
@@ -455,13 +493,15 @@ __global__ __launch_bounds__(256) void k_apc_final(const float *__restrict__ M, 
     }
 }
 
-hipError_t launch_apc_finalize(const float *M, const float *r, float *coef, const float *w_dev, int LH, SeqMeta sm,
-                               float bias, float *contacts, int n_stride, hipStream_t st) {
+hipError_t launch_apc_finalize(const float *M, const float *r, float *coef, const float *w_dev, const int *lhs_dev,
+                               int nlh, SeqMeta sm, float bias, float *contacts, int n_stride, hipStream_t st) {
     if (sm.S_max < 3) return hipSuccess;
     const int n_max = sm.S_max - 2;
-    hipLaunchKernelGGL(k_apc_coef, dim3(LH, sm.B), dim3(256), 0, st, r, w_dev, sm.lens, sm.S_max, sm.B, coef);
+    if (nlh > 0)
+        hipLaunchKernelGGL(k_apc_coef, dim3(nlh, sm.B), dim3(256), 0, st, r, w_dev, lhs_dev, sm.lens, sm.S_max, sm.B,
+                           coef);
     const int nt = (n_max + APC_FT - 1) / APC_FT;
-    hipLaunchKernelGGL(k_apc_final, dim3(nt, nt, sm.B), dim3(256), 0, st, M, r, coef, LH, sm.lens, sm.S_max, sm.B, bias,
+    hipLaunchKernelGGL(k_apc_final, dim3(nt, nt, sm.B), dim3(256), 0, st, M, r, coef, lhs_dev, nlh, sm.lens, sm.S_max, sm.B, bias,
                        contacts, n_stride);
     return hipGetLastError();
 }

@@ -100,8 +100,10 @@ struct cih_model {
     float contact_b = 0.0f;
     bool has_contacts = false;
     float *d_contact_w = nullptr;
-    int *d_heads = nullptr;  // [L][H] per-layer list of heads with nonzero weight
+    int *d_heads = nullptr;  // [L][H] per layer: the nz[l] heads with nonzero weight, then the others
     std::vector<int> nz;
+    int *d_lhs = nullptr;  // the n_lhs layer-heads l H + h of nonzero weight, in order
+    int n_lhs = 0;
     cih::Workspace ws;
     cih::Prof prof;
 };

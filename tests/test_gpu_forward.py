@@ -109,6 +109,35 @@ def test_forward_small_configs(hd, H, dtype, act, monkeypatch):
     check_batch(cfg, w, seqs, ALL, contact=(cw, np.float32(-0.5)))
 
 
+@pytest.mark.parametrize("dtype,lens", [(1, [8]), (1, [33]), (2, [97, 40, 3]), (0, [260, 1, 130, 222, 31]),
+                                        (1, [700, 555, 641, 2, 300])])
+@pytest.mark.parametrize("H,hd", [(24, 16), (20, 24), (20, 32), (8, 64)])
+def test_contacts_sparse_heads(H, hd, dtype, lens):
+    """Heads of zero contact weight (most of ESM-2's) skip the probability export: per layer 0, 1, 2, 4, 7, 12 and
+    20 heads in use (as H allows), on the few-token, wave-split, staged and tile-image attention.  Checked against the
+    oracle, and against the route that exports every head (the zeros replaced by weights too small to count): the
+    two softmax forms agree to FP32 rounding (1e-6 of a probability, weighted and summed over the heads)."""
+    counts = [0, 1, 2, 4, min(7, H), min(12, H), min(20, H)]
+    cfg = ch.EsmConfig(H * hd, 2 * H * hd // 32 * 32, len(counts), H)
+    w = quantized(ch.EsmWeights.random(cfg, seed=H + hd, std=0.05, bias_std=0.02), dtype)
+    rng = np.random.default_rng(17 * H + hd)
+    head = np.zeros((len(counts), H), np.float32)
+    for row, n in zip(head, counts):
+        row[rng.permutation(H)[:n]] = rng.normal(0, 3, n)
+    seqs = [rand_tokens(rng, max(n - 2, 0))[:n] for n in lens]
+    flags = ch.OUT_LOGITS | ch.OUT_CONTACTS
+    check_batch(cfg, w, seqs, flags, contact=(head, np.float32(-1.0)))
+    got = []
+    for weights in (head, np.where(head == 0, np.float32(1e-30), head)):
+        m = ch.GpuModel(cfg, w, contact_head=(weights, np.float32(-1.0)), max_batch=len(seqs),
+                        max_len=max(lens), outputs=flags)
+        got.append(m.forward(seqs, flags))
+        m.close()
+    scale = 1e-6 * float(np.abs(head).sum())
+    assert np.abs(got[0]["contacts"] - got[1]["contacts"]).max() <= scale
+    assert np.abs(got[0]["logits"] - got[1]["logits"]).max() <= 1e-5 * max(1.0, np.abs(got[1]["logits"]).max())
+
+
 def test_contacts_forty_heads():
     """Contacts with more than 20 weighted heads per layer (the 3B and 15B
     head count, 40): the map reader's 40-head pass, with a few zero-weight
