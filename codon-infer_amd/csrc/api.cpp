@@ -42,7 +42,7 @@ std::string kernel_switches() {
                                         "CIH_GEMV_NB", "CIH_GEMM_LDS", "CIH_GEMM_TILE", "CIH_GEMM_TILE_N",
                                         "CIH_GEMM_TILE_N_GELU", "CIH_ATT_IMG", "CIH_GEMV16", "CIH_GEMV16_KW",
                                         "CIH_FEW_WO", "CIH_DECODE_LN", "CIH_ATT_XCD", "CIH_GEMM_SCHED",
-                                        "CIH_GEMM_PLAN", "CIH_GEMM_PERSIST", "CIH_GEMM_KW"};
+                                        "CIH_GEMM_PLAN", "CIH_GEMM_PERSIST", "CIH_GEMM_KW", "CIH_GEMM_ROWS"};
     std::string s = g_full_range ? "R|" : "|";
     for (const char *n : names) {
         const char *v = getenv(n);
@@ -124,6 +124,33 @@ namespace {
 }  // namespace
 
 namespace cih {
+
+// How T rows' activations reach the layer projections: FP32, three bf16 limbs
+// or two f16 limbs (see forward_impl).
+int activation_format(const cih_model *m, int T) {
+    const int d = m->cfg.dim, F = m->cfg.hidden_dim, L = m->cfg.n_layers;
+    int af = AF_F32;
+    const char *qpath = getenv("CIH_QGEMM"), *apath = getenv("CIH_ACT"), *lpath = getenv("CIH_LIMBS");
+    const bool fp32_gemm = qpath && !std::strcmp(qpath, "fp32");
+    const bool bf16 = lpath && !std::strcmp(lpath, "bf16x3");
+    if (m->dtype != DT_FP32 && !fp32_gemm && T > GEMV_MAX_M) {
+        if ((apath && !std::strcmp(apath, "x3")) || full_range_mode()) af = AF_X3;
+        else if (!(apath && !std::strcmp(apath, "f32")) && !bf16) af = AF_H2;
+    } else if (m->dtype == DT_FP32 && !fp32_gemm && !bf16 && !apath && !full_range_mode() && T > GEMV_MAX_M &&
+               L > 0 && m->layers[0].wqkv.p16) {
+        // FP32 weights through their f16 pair copies: the activations as
+        // f16 limbs too (the same split the GEMM makes of FP32 ones, so the
+        // same bits), which the LDS-staged GEMM reads; CIH_ACT=f32: FP32
+        af = AF_H2;
+    } else if (m->dtype != DT_FP32 && !fp32_gemm && !apath && !bf16 && !full_range_mode() && L > 0 &&
+               gemv16_applies(m->layers[0].wqkv, AF_H2, T, EPI_NONE) &&
+               gemv16_applies(m->layers[0].wo, AF_H2, T, EPI_NONE) &&
+               gemv16_applies(m->layers[0].w1, AF_H2, T, EPI_NONE) &&
+               gemv16_applies(m->layers[0].w2, AF_H2, T, EPI_NONE) && d % 32 == 0 && F % 32 == 0) {
+        af = AF_H2;  // few tokens: the f16-MFMA GEMV (k_gemv16) reads limbs
+    }
+    return af;
+}
 
 hipError_t model_gemm(cih_model *m, const PartialBuf &pb, const DevMatrix &W, const void *X, int ldx, int a_fmt,
                       const float *bias, void *Y, int ldy, int M, int epi, int *defer) {
@@ -380,28 +407,7 @@ int forward_impl(cih_model *m, const int32_t *tokens, const int32_t *lens, int32
     // CIH_QGEMM=fp32 imply FP32 hand-off.  Batches of at most GEMV_MAX_M
     // tokens take the f16-MFMA GEMV (k_gemv16), which reads limbs too; with
     // any of those switches, CIH_GEMV16=0 or in full range the FP32 GEMV.
-    int af = AF_F32;
-    {
-        const char *qpath = getenv("CIH_QGEMM"), *apath = getenv("CIH_ACT"), *lpath = getenv("CIH_LIMBS");
-        const bool fp32_gemm = qpath && !std::strcmp(qpath, "fp32");
-        const bool bf16 = lpath && !std::strcmp(lpath, "bf16x3");
-        if (m->dtype != DT_FP32 && !fp32_gemm && T > GEMV_MAX_M) {
-            if ((apath && !std::strcmp(apath, "x3")) || full_range_mode()) af = AF_X3;
-            else if (!(apath && !std::strcmp(apath, "f32")) && !bf16) af = AF_H2;
-        } else if (m->dtype == DT_FP32 && !fp32_gemm && !bf16 && !apath && !full_range_mode() && T > GEMV_MAX_M &&
-                   L > 0 && m->layers[0].wqkv.p16) {
-            // FP32 weights through their f16 pair copies: the activations as
-            // f16 limbs too (the same split the GEMM makes of FP32 ones, so the
-            // same bits), which the LDS-staged GEMM reads; CIH_ACT=f32: FP32
-            af = AF_H2;
-        } else if (m->dtype != DT_FP32 && !fp32_gemm && !apath && !bf16 && !full_range_mode() && L > 0 &&
-                   gemv16_applies(m->layers[0].wqkv, AF_H2, T, EPI_NONE) &&
-                   gemv16_applies(m->layers[0].wo, AF_H2, T, EPI_NONE) &&
-                   gemv16_applies(m->layers[0].w1, AF_H2, T, EPI_NONE) &&
-                   gemv16_applies(m->layers[0].w2, AF_H2, T, EPI_NONE) && d % 32 == 0 && F % 32 == 0) {
-            af = AF_H2;  // few tokens: the f16-MFMA GEMV (k_gemv16) reads limbs
-        }
-    }
+    const int af = activation_format(m, T);
     const int epi_fc1 = af == AF_X3 ? EPI_GELU_X3 : (af == AF_H2 ? EPI_GELU_H2 : EPI_GELU);
     // Few tokens (af == AF_H2 at T <= GEMV_MAX_M: the f16-MFMA GEMV): each
     // projection leaves split-K partial sums in one half of the partial
@@ -642,7 +648,7 @@ int forward_impl(cih_model *m, const int32_t *tokens, const int32_t *lens, int32
     // and an output the LM head's limbs cannot hold.  Without a hidden-state
     // export it hands the LM head's dense layer (FP32 weights through their
     // pair copy) f16 limbs: the split that GEMM makes of FP32 rows, so the
-    // same bits, and from 64 rows on the LDS-staged kernel reads them.
+    // same bits, and k_gemm_rows or the LDS-staged kernel reads them.
     const bool lm_h2 = (want_logits || keep_logits) && m->has_head && !want_hidden && af == AF_H2 &&
                        T > GEMV_MAX_M && m->dense.fmt == WF_F32 && m->dense.p16 && m->dense.psc && d % 32 == 0;
     {

@@ -164,11 +164,21 @@ int enqueue_rows(cih_decoder *dc, int n, bool fused) {
             pend_bias = ly.b2;
         }
     }
+    // More rows than the GEMV takes: the activations travel as f16 limbs (as in
+    // the bidirectional forward), written by the LayerNorms, the attention and
+    // FC1, and split residual projections leave their sums to the LayerNorm
+    // after them.  Full range and the switches of the GEMMs keep FP32.
+    const bool h2 = n > GEMV_MAX_M && d % 32 == 0 && d <= 8192 && activation_format(m, n) == AF_H2;
+    const int af = h2 ? AF_H2 : AF_F32;
     for (int l = 0; l < L && !g16; l++) {
         const Layer &ly = m->layers[l];
         {
             ProfScope ps(m, CIH_KC_OTHER, 0, 8.0 * n * d);
-            HIPCHK(launch_layernorm(dc->x, ly.ln1w, ly.ln1b, dc->xb, AF_F32, n, d, st));
+            if (pend_splits)
+                HIPCHK(launch_residual_layernorm(dc->x, part_a, pend_splits, pend_bias, ly.ln1w, ly.ln1b, dc->xb, af, n,
+                                                 d, st));
+            else
+                HIPCHK(launch_layernorm(dc->x, ly.ln1w, ly.ln1b, dc->xb, af, n, d, st));
         }
         // one row per sequence through the GEMV: the attention kernel adds
         // the QKV partial sums itself (no separate reduction)
@@ -179,7 +189,7 @@ int enqueue_rows(cih_decoder *dc, int n, bool fused) {
                          wbytes(ly.wqkv) + 4.0 * n * d + 4.0 * n * ly.wqkv.N);
             HIPCHK(launch_gemv_partials(ly.wqkv, dc->xb, d, n, dc->part, &splits, st));
         } else {
-            HIPCHK(model_gemm(m, dc->part, ly.wqkv, dc->xb, d, AF_F32, ly.bqkv, dc->qkv, 3 * d, n, EPI_NONE));
+            HIPCHK(model_gemm(m, dc->part, ly.wqkv, dc->xb, d, af, ly.bqkv, dc->qkv, 3 * d, n, EPI_NONE));
         }
         float *kc = dc->kc + l * layer, *vc = dc->vc + l * layer;
         {
@@ -188,21 +198,27 @@ int enqueue_rows(cih_decoder *dc, int n, bool fused) {
             if (fused) {
                 HIPCHK(launch_decode_attention_fused(dc->qkv, qkv_parts ? dc->part.part : nullptr, splits, ly.bqkv, d,
                                                      H, dc->d_rows, n, dc->max_len, dc->rope_c, dc->rope_s, kc, vc,
-                                                     dc->slot_stride, dc->ao, st));
+                                                     dc->slot_stride, dc->ao, st, af));
             } else {
                 HIPCHK(launch_rope_kv(dc->qkv, d, m->hd, dc->d_rows, n, dc->rope_c, dc->rope_s, kc, vc,
                                       dc->slot_stride, st));
                 HIPCHK(launch_decode_attention(dc->qkv, d, H, dc->d_rows, n, dc->max_len, kc, vc, dc->slot_stride,
-                                               dc->ao, st));
+                                               dc->ao, st, af));
             }
         }
-        HIPCHK(model_gemm(m, dc->part, ly.wo, dc->ao, d, AF_F32, ly.bo, dc->x, d, n, EPI_RESIDUAL));
+        int so = 0, s2 = 0;
+        HIPCHK(model_gemm(m, dc->part, ly.wo, dc->ao, d, af, ly.bo, dc->x, d, n, EPI_RESIDUAL, h2 ? &so : nullptr));
         {
-            ProfScope ps(m, CIH_KC_OTHER, 0, 8.0 * n * d);
-            HIPCHK(launch_layernorm(dc->x, ly.ln2w, ly.ln2b, dc->xb, AF_F32, n, d, st));
+            ProfScope ps(m, CIH_KC_OTHER, 0, 8.0 * n * d + 4.0 * so * n * d);
+            if (so)
+                HIPCHK(launch_residual_layernorm(dc->x, part_a, so, ly.bo, ly.ln2w, ly.ln2b, dc->xb, af, n, d, st));
+            else
+                HIPCHK(launch_layernorm(dc->x, ly.ln2w, ly.ln2b, dc->xb, af, n, d, st));
         }
-        HIPCHK(model_gemm(m, dc->part, ly.w1, dc->xb, d, AF_F32, ly.b1, dc->h, F, n, EPI_GELU));
-        HIPCHK(model_gemm(m, dc->part, ly.w2, dc->h, F, AF_F32, ly.b2, dc->x, d, n, EPI_RESIDUAL));
+        HIPCHK(model_gemm(m, dc->part, ly.w1, dc->xb, d, af, ly.b1, dc->h, F, n, h2 ? EPI_GELU_H2 : EPI_GELU));
+        HIPCHK(model_gemm(m, dc->part, ly.w2, dc->h, F, af, ly.b2, dc->x, d, n, EPI_RESIDUAL, h2 ? &s2 : nullptr));
+        pend_splits = s2;
+        pend_bias = ly.b2;
     }
     {
         // more rows than the GEMV takes go through GEMMs on f16 limbs: the

@@ -1297,7 +1297,8 @@ hipError_t launch_gemm_lds_split(const DevMatrix &W, const void *X, int M, const
 // Routing of the problems that do not fill the device with 128-row tiles,
 // from a sweep of every tile and split over the ESM-2 8M-3B projections at
 // 16-8192 tokens on MI355X (256 CUs; the thresholds scale with the CU
-// count); below 64 rows the register-staged kernel stays.  One 4-wave workgroup per CU exposes the per-block barrier and
+// count); below 49 rows k_gemm_rows (49 to 63 rows read a
+// 64-row tile past their end, clamped: as fast as at 64).  One 4-wave workgroup per CU exposes the per-block barrier and
 // operand-read latency to its lone wave per SIMD; smaller tiles put three or
 // four workgroups on each CU and leave fewer CUs idle in the last round.  A
 // split's partial sums cost the LayerNorm that adds them about S M N 4 bytes
@@ -1324,7 +1325,7 @@ bool gemm_lds_plan(const DevMatrix &W, int a_fmt, int M, int epi, size_t part_fl
         W.N <= 0 || W.kx % 32)
         return false;
     if (epi != EPI_NONE && epi != EPI_RESIDUAL && epi != EPI_GELU_H2 && !(epi == EPI_GELU && W.kx)) return false;
-    if (M < 64) return false;  // fewer rows: the register-staged kernel (and its splits) is as fast or faster
+    if (M <= 48) return false;  // fewer rows: k_gemm_rows
     const char *le = getenv("CIH_GEMM_LDS"), *pe = getenv("CIH_GEMM_PLAN"), *ke = getenv("CIH_SPLITK");
     if (le || (pe && !strcmp(pe, "0"))) return false;  // CIH_GEMM_LDS=0 / force: the routes without the plan
     const long cus = device_cus();

@@ -582,7 +582,9 @@ hipError_t launch_gemm_x3(const DevMatrix &W, const void *X, int ldx, int a_fmt,
     if (M <= 0) return hipSuccess;
     if (W.K % 32 != 0 || (a_fmt == AF_F32 && ldx % 4 != 0)) return hipErrorInvalidValue;
     if ((epi == EPI_GELU_X3 || epi == EPI_GELU_H2) && W.N % 32 != 0) return hipErrorInvalidValue;
-    // f16 limbs with the f16 copy of the quants, 64 rows and more: the LDS
+    if (gemm_rows_applies(W, a_fmt, M, epi))
+        return launch_gemm_rows(W, static_cast<const unsigned short *>(X), bias, Y, ldy, M, epi, pb, defer, st);
+    // f16 limbs with the f16 copy of the quants, 49 rows and more: the LDS
     // kernel's tile (and split) for the shape.  An FP32 matrix's pair copy
     // (W.q: [2K/32][N][32] f16) goes the same way as an f16 matrix of 2K
     // whose block kb meets activation block kb mod K/32.

@@ -185,6 +185,16 @@ hipError_t launch_gemm(const DevMatrix &W, const void *X, int ldx, int a_fmt, co
 hipError_t launch_gemm_x3(const DevMatrix &W, const void *X, int ldx, int a_fmt, const float *bias, void *Y,
                           int ldy, int M, int epi, const PartialBuf *pb, hipStream_t st, int *defer = nullptr);
 
+// The same GEMM for a few dozen rows (gemm_rows.hip): f16-limb activations, W
+// in Q8_0 / Q4_0 or a pair copy (WF_F16P, K the activations' length).  A
+// residual projection with defer may leave K splits [S][M][N] in pb for the
+// caller to add (*defer = S, 0 when the epilogue was applied).
+// CIH_GEMM_ROWS=0 turns it off.
+constexpr int GEMM_ROWS_MAX = 64;
+bool gemm_rows_applies(const DevMatrix &W, int a_fmt, int M, int epi);
+hipError_t launch_gemm_rows(const DevMatrix &W, const unsigned short *X, const float *bias, void *Y, int ldy, int M,
+                            int epi, const PartialBuf *pb, int *defer, hipStream_t st);
+
 // Weight-streaming GEMV for M <= GEMV_MAX_M tokens (FP32 activations, epilogue
 // EPI_NONE / EPI_GELU / EPI_RESIDUAL).  With several k-splits the partial sums
 // go through pb ([splits][M][N] floats) and a second kernel.
@@ -245,7 +255,7 @@ hipError_t launch_to_h2(const float *x, int M, int K, unsigned short *out, hipSt
 // global -> LDS by the load unit (no staging registers), W read from W.q16
 // or, without it, from the quants.  Epilogues EPI_NONE / EPI_RESIDUAL /
 // EPI_GELU_H2 (and the QKV image epilogues).  With W.q16, launch_gemm_x3
-// routes f16-limb calls of 64 rows and more by gemm_lds_plan (below);
+// routes f16-limb calls of 49 rows and more by gemm_lds_plan (below);
 // otherwise gemm_lds_applies says whether it routes a call here: the shape
 // must give at least one full round of 128x128 tiles (smaller problems keep
 // the split-K path).  CIH_GEMM_LDS=0 never, =force whenever the formats
@@ -262,7 +272,7 @@ hipError_t launch_gemm_lds_split(const DevMatrix &W, const void *X, int M, const
                                  hipStream_t st);
 // Workgroup tiles of the LDS-staged GEMM (BM x BN).
 enum LdsTileId { LDS_TILE_128x128 = 1, LDS_TILE_128x160, LDS_TILE_128x256, LDS_TILE_128x320, LDS_TILE_64x128, LDS_TILE_64x64 };
-// Tile and k-splits for an f16-limb GEMM with the f16 copy from 64 rows on
+// Tile and k-splits for an f16-limb GEMM with the f16 copy from 49 rows on
 // (false: not such a GEMM, or CIH_GEMM_LDS / CIH_GEMM_PLAN=0 set).  Splits
 // only for EPI_RESIDUAL with room for them (part_floats > 0; the caller
 // adds them, as launch_gemm_lds_split's).  kw: groups of 4 waves that share
