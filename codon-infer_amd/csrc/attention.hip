@@ -806,6 +806,10 @@ __global__ __launch_bounds__(NTH, ONEPASS || HD <= 32 ? 4 : 2) void k_attention_
 // Per query the arithmetic is k_attention_h's, with the softmax and P.V sums
 // regrouped by wave: agreement to rounding, not bit for bit.
 // MODE: ATT_ONEPASS, ATT_EXPORT, or ATT_MIXED (head slots below nexp export).
+// Latency-bound: KS is 2 or 4 where the sequences have no more tiles (fewer
+// sums to join), each tile is requested before the work ahead of it, and the
+// output's sums are shared by the waves.  650M, one 41-token sequence: 12.2 ->
+// 8.6 us per layer.
 template <int HD, int KS, int MODE>
 __global__ __launch_bounds__(64 * KS) void k_attention_xs(const float *__restrict__ qkv, int d,
                                                           const int *__restrict__ cu, const int *__restrict__ lens,
@@ -862,6 +866,85 @@ __global__ __launch_bounds__(64 * KS) void k_attention_xs(const float *__restric
             Vl[c * V_LD + key] = (_Float16)0.0f;
         }
 
+    // K tile: a lane rotates 4 consecutive pair-dims (c..c+3 with c+HALF..) of
+    // one key.  V tile, transposed: a lane takes 4 consecutive keys of one dim.
+    // fetch_* requests a tile into registers, stage_* turns it into limbs in
+    // the wave's LDS: a wave's first tile is requested before the query is
+    // read, a later one before its predecessor is computed.
+    constexpr int KG = HALF / 4, KI = (32 * KG + 63) / 64, VI = (8 * HD + 63) / 64;
+    f32x4 kr[KI][4], vr[VI];
+    auto fetch_k = [&](int kt0) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < KI; i++) {
+            const int idx = min(lane + 64 * i, 32 * KG - 1);
+            const int key = idx / KG, c = 4 * (idx % KG);
+            const int kk = min(kt0 + key, len - 1);
+            const float *krow = Kg + (size_t)(base + kk) * ld;
+            kr[i][0] = *reinterpret_cast<const f32x4 *>(krow + c);
+            kr[i][1] = *reinterpret_cast<const f32x4 *>(krow + c + HALF);
+            kr[i][2] = *reinterpret_cast<const f32x4 *>(rc + (size_t)kk * HALF + c);
+            kr[i][3] = *reinterpret_cast<const f32x4 *>(rsn + (size_t)kk * HALF + c);
+        }
+    };
+    auto stage_k = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < KI; i++) {
+            const int idx = lane + 64 * i;
+            if (32 * KG % 64 != 0 && idx >= 32 * KG) break;
+            const int key = idx / KG, c = 4 * (idx % KG);
+            const f32x4 k0 = kr[i][0], k1 = kr[i][1], cs = kr[i][2], sn = kr[i][3];
+            f16x4 h0, l0, h1, l1;
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const float r0 = rot_lo(k0[e], k1[e], cs[e], sn[e]);
+                const float r1 = rot_hi(k1[e], k0[e], cs[e], sn[e]);
+                h0[e] = (_Float16)r0;
+                l0[e] = (_Float16)(r0 - (float)h0[e]);
+                h1[e] = (_Float16)r1;
+                l1[e] = (_Float16)(r1 - (float)h1[e]);
+            }
+            *reinterpret_cast<f16x4 *>(&Kh[key * K_LD + c]) = h0;
+            *reinterpret_cast<f16x4 *>(&Kl[key * K_LD + c]) = l0;
+            *reinterpret_cast<f16x4 *>(&Kh[key * K_LD + c + HALF]) = h1;
+            *reinterpret_cast<f16x4 *>(&Kl[key * K_LD + c + HALF]) = l1;
+        }
+    };
+    auto fetch_v = [&](int kt0) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < VI; i++) {
+            const int idx = min(lane + 64 * i, 8 * HD - 1);
+            const int c = idx % HD, kg = 4 * (idx / HD);
+#pragma unroll
+            for (int e = 0; e < 4; e++) vr[i][e] = Vg[(size_t)(base + min(kt0 + kg + e, len - 1)) * ld + c];
+        }
+    };
+    auto stage_v = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < VI; i++) {
+            const int idx = lane + 64 * i;
+            if (8 * HD % 64 != 0 && idx >= 8 * HD) break;
+            const int c = idx % HD, kg = 4 * (idx / HD);
+            f16x4 hv, lv;
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const float v = vr[i][e];
+                hv[e] = (_Float16)v;
+                lv[e] = (_Float16)(v - (float)hv[e]);
+            }
+            const int pos = (kg & ~15) | ((kg & 4) << 1) | ((kg & 8) >> 1);  // as in k_attention_h
+            *reinterpret_cast<f16x4 *>(&Vh[c * V_LD + pos]) = hv;
+            *reinterpret_cast<f16x4 *>(&Vl[c * V_LD + pos]) = lv;
+        }
+    };
+    const int ntile = (len + 31) / 32;
+    // the mixed form holds both softmax bodies: V is fetched when it is staged
+    // there (the early request spills)
+    constexpr bool EARLY_V = MODE != ATT_MIXED || HD < 64;
+    if (w < ntile) {
+        fetch_k(w * 32);
+        if (EARLY_V) fetch_v(w * 32);
+    }
+
     // rotated query dims 16c + 8hh + e of this lane's query, as f16 limbs
     const float sl2 = inv_scale * 1.44269504088896340736f;
     const int qi = qblk + li;
@@ -879,64 +962,12 @@ __global__ __launch_bounds__(64 * KS) void k_attention_xs(const float *__restric
                 float r = 0.0f;
                 if (dim < HALF) r = rot_lo(qrow[dim], qrow[dim + HALF], cs[dim], sn[dim]);
                 else if (dim < HD) r = rot_hi(qrow[dim], qrow[dim - HALF], cs[dim - HALF], sn[dim - HALF]);
-                v[e] = opaque(r * sl2);  // pre-scaled, as in k_attention_h
+                v[e] = opaque(r * sl2);
             }
             split8(v, qh[c], ql[c]);
         }
     }
 
-    // K tile: a lane rotates 4 consecutive pair-dims (c..c+3 with c+HALF..) of one key
-    auto load_k = [&](int kt0) __attribute__((always_inline)) {
-        constexpr int G = HALF / 4;
-#pragma unroll
-        for (int i = 0; i < (32 * G + 63) / 64; i++) {
-            const int idx = lane + 64 * i;
-            if (32 * G % 64 != 0 && idx >= 32 * G) break;
-            const int key = idx / G, c = 4 * (idx % G);
-            const int kk = min(kt0 + key, len - 1);
-            const float *krow = Kg + (size_t)(base + kk) * ld;
-            const float4 k0 = *reinterpret_cast<const float4 *>(krow + c);
-            const float4 k1 = *reinterpret_cast<const float4 *>(krow + c + HALF);
-            const float4 cs = *reinterpret_cast<const float4 *>(rc + (size_t)kk * HALF + c);
-            const float4 sn = *reinterpret_cast<const float4 *>(rsn + (size_t)kk * HALF + c);
-            const float r0[4] = {rot_lo(k0.x, k1.x, cs.x, sn.x), rot_lo(k0.y, k1.y, cs.y, sn.y),
-                                 rot_lo(k0.z, k1.z, cs.z, sn.z), rot_lo(k0.w, k1.w, cs.w, sn.w)};
-            const float r1[4] = {rot_hi(k1.x, k0.x, cs.x, sn.x), rot_hi(k1.y, k0.y, cs.y, sn.y),
-                                 rot_hi(k1.z, k0.z, cs.z, sn.z), rot_hi(k1.w, k0.w, cs.w, sn.w)};
-            f16x4 h0, l0, h1, l1;
-#pragma unroll
-            for (int e = 0; e < 4; e++) {
-                h0[e] = (_Float16)r0[e];
-                l0[e] = (_Float16)(r0[e] - (float)h0[e]);
-                h1[e] = (_Float16)r1[e];
-                l1[e] = (_Float16)(r1[e] - (float)h1[e]);
-            }
-            *reinterpret_cast<f16x4 *>(&Kh[key * K_LD + c]) = h0;
-            *reinterpret_cast<f16x4 *>(&Kl[key * K_LD + c]) = l0;
-            *reinterpret_cast<f16x4 *>(&Kh[key * K_LD + c + HALF]) = h1;
-            *reinterpret_cast<f16x4 *>(&Kl[key * K_LD + c + HALF]) = l1;
-        }
-    };
-    // V tile, transposed: a lane takes 4 consecutive keys of one dim
-    auto load_v = [&](int kt0) __attribute__((always_inline)) {
-#pragma unroll
-        for (int i = 0; i < (8 * HD + 63) / 64; i++) {
-            const int idx = lane + 64 * i;
-            if (8 * HD % 64 != 0 && idx >= 8 * HD) break;
-            const int c = idx % HD, kg = 4 * (idx / HD);
-            f16x4 hv, lv;
-#pragma unroll
-            for (int e = 0; e < 4; e++) {
-                const int kk = min(kt0 + kg + e, len - 1);
-                const float v = Vg[(size_t)(base + kk) * ld + c];
-                hv[e] = (_Float16)v;
-                lv[e] = (_Float16)(v - (float)hv[e]);
-            }
-            const int pos = (kg & ~15) | ((kg & 4) << 1) | ((kg & 8) >> 1);  // as in k_attention_h
-            *reinterpret_cast<f16x4 *>(&Vh[c * V_LD + pos]) = hv;
-            *reinterpret_cast<f16x4 *>(&Vl[c * V_LD + pos]) = lv;
-        }
-    };
     auto scores = [&](f32x16 &acc, float c0) __attribute__((always_inline)) {
 #pragma unroll
         for (int q = 0; q < 16; q++) acc[q] = c0;
@@ -967,15 +998,15 @@ __global__ __launch_bounds__(64 * KS) void k_attention_xs(const float *__restric
         }
     };
 
-    const int ntile = (len + 31) / 32;
     float *ox = reinterpret_cast<float *>(sm);
     // The waves' P.V accumulators (scaled by f) added in wave order and stored
-    // for this lane's query, times out_scale; every wave must have written ox.
+    // for this lane's query, times out_scale; every wave must have written ox
+    // and takes every KS-th group of four output dims.
     auto finish = [&](float out_scale) __attribute__((always_inline)) {
         if (qi >= len) return;
         // output dims t 32 + 8 g + 4 hh + {0..3}: registers 4 g + {0..3} of tile t
 #pragma unroll 1
-        for (int tg = 0; tg < 4 * DT; tg++) {
+        for (int tg = w; tg < 4 * DT; tg += KS) {
             const int t = tg >> 2, g = tg & 3;
             const int dd = t * 32 + 8 * g + 4 * hh;
             if (dd >= HD) continue;
@@ -1013,9 +1044,14 @@ __global__ __launch_bounds__(64 * KS) void k_attention_xs(const float *__restric
         for (int t = w; t < ntile; t += KS) {
             const int kt0 = t * 32;
             wave_sync();
-            load_k(kt0);
-            load_v(kt0);
+            stage_k();
+            if (!EARLY_V) fetch_v(kt0);
+            stage_v();
             wave_sync();
+            if (t + KS < ntile) {
+                fetch_k(kt0 + 32 * KS);
+                if (EARLY_V) fetch_v(kt0 + 32 * KS);
+            }
             if (kt0 + 32 <= len) tile(kt0, std::false_type{});
             else tile(kt0, std::true_type{});
         }
@@ -1038,7 +1074,7 @@ __global__ __launch_bounds__(64 * KS) void k_attention_xs(const float *__restric
 #pragma unroll
             for (int q = 0; q < 16; q++) ox[((w * DT + t) * 16 + q) * 64 + lane] = f * oacc[t][q];
         __syncthreads();
-        if (w == 0) finish(1.0f / L);
+        finish(1.0f / L);
         return;
     }
     if constexpr (MODE != ATT_ONEPASS) {
@@ -1047,8 +1083,9 @@ __global__ __launch_bounds__(64 * KS) void k_attention_xs(const float *__restric
         for (int t = w; t < ntile; t += KS) {
             const int kt0 = t * 32;
             wave_sync();
-            load_k(kt0);
+            stage_k();
             wave_sync();
+            if (ntile > KS) fetch_k((t + KS < ntile ? t + KS : w) * 32);  // (the last one: pass 2's first)
             f32x16 acc;
             scores(acc, 0.0f);
             float sv[16];
@@ -1097,9 +1134,14 @@ __global__ __launch_bounds__(64 * KS) void k_attention_xs(const float *__restric
         for (int t = w; t < ntile; t += KS) {
             const int kt0 = t * 32;
             wave_sync();
-            load_k(kt0);
-            load_v(kt0);
+            if (ntile > KS) stage_k();  // (one tile per wave: still staged from pass 1)
+            if (!EARLY_V) fetch_v(kt0);
+            stage_v();
             wave_sync();
+            if (t + KS < ntile) {
+                fetch_k(kt0 + 32 * KS);
+                if (EARLY_V) fetch_v(kt0 + 32 * KS);
+            }
             f32x16 acc;
             scores(acc, 0.0f);
             float p[16];
@@ -1119,11 +1161,12 @@ __global__ __launch_bounds__(64 * KS) void k_attention_xs(const float *__restric
 #pragma unroll
             for (int q = 0; q < 16; q++) ox[((w * DT + t) * 16 + q) * 64 + lane] = oacc[t][q];
         __syncthreads();
-        if (w != 0) return;
-        float rsum = red[0][2][lane];
+        if (w == 0) {
+            float rsum = red[0][2][lane];
 #pragma unroll
-        for (int s = 1; s < KS; s++) rsum += red[s][2][lane];
-        write_rowsum(rowsum, rsum, b, h, H, S_max, qi, len, hh);
+            for (int s = 1; s < KS; s++) rsum += red[s][2][lane];
+            write_rowsum(rowsum, rsum, b, h, H, S_max, qi, len, hh);
+        }
         finish(1.0f);
     }
 }
@@ -1626,10 +1669,16 @@ hipError_t launch_attention(const float *qkv, int d, int H, SeqMeta sm, const fl
     hipLaunchKernelGGL((k_attention_h<HDV, ONE, NTH>), dim3(grid), dim3(NTH), 0, st, qkv, d, sm.cu, sm.lens,     \
                        sm.S_max, rope_cos, rope_sin, out, out_fmt, P, (long long)pb, (long long)ph, inv_scale, rowsum, \
                        H, nq, nfull, nsplit, part, order, nexp)
-#define CIH_ATT_XS(HDV, MODE)                                                                                   \
-    hipLaunchKernelGGL((k_attention_xs<HDV, 8, MODE>), dim3(t32), dim3(512), 0, st, qkv, d, sm.cu, sm.lens,      \
+#define CIH_ATT_XSK(HDV, KS, MODE)                                                                              \
+    hipLaunchKernelGGL((k_attention_xs<HDV, KS, MODE>), dim3(t32), dim3(64 * KS), 0, st, qkv, d, sm.cu, sm.lens, \
                        sm.S_max, rope_cos, rope_sin, out, out_fmt, P, (long long)pb, (long long)ph, inv_scale,   \
                        rowsum, H, nq32, order, nexp)
+#define CIH_ATT_XS(HDV, MODE)                                                                                   \
+    do {                                                                                                        \
+        if (nq32 <= 2) CIH_ATT_XSK(HDV, 2, MODE);                                                               \
+        else if (nq32 <= 4) CIH_ATT_XSK(HDV, 4, MODE);                                                          \
+        else CIH_ATT_XSK(HDV, 8, MODE);                                                                         \
+    } while (0)
 #define CIH_ATT(HDV)                                                                                           \
     if (xsplit && mixed) CIH_ATT_XS(HDV, ATT_MIXED);                                                            \
     else if (xsplit && P) CIH_ATT_XS(HDV, ATT_EXPORT);                                                          \
@@ -1657,6 +1706,7 @@ hipError_t launch_attention(const float *qkv, int d, int H, SeqMeta sm, const fl
 #undef CIH_ATT
 #undef CIH_ATT_H
 #undef CIH_ATT_XS
+#undef CIH_ATT_XSK
 #undef CIH_ATT_K
     return hipGetLastError();
 }
