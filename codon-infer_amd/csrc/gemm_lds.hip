@@ -1108,7 +1108,8 @@ hipError_t launch_t(const DevMatrix &W, const void *X, const float *bias, void *
 }
 
 // Split-K form: grid (tiles, S), raw partial sums into part.  128 x 128 tiles
-// (4 waves) for every weight form; 64 x 128 and 64 x 64 from the f16 copy.
+// (4 waves) for every weight form; 128 x 320, 64 x 128 and 64 x 64 from the
+// f16 copy.
 template <int RT, int CT, int WM, int WN, int KW = 1>
 hipError_t launch_split_t(const DevMatrix &W, const void *X, int M, float *part, int S, int kps, hipStream_t st) {
     using T = LdsTile<RT, CT, WM, WN>;
@@ -1128,6 +1129,16 @@ hipError_t launch_split_t(const DevMatrix &W, const void *X, int M, float *part,
             hipLaunchKernelGGL((k_gemm_lds<EPI_NONE, RT, CT, WM, WN, 0, true, 0, false, false, KW>), grid, block, 0, st,
                                Xh, reinterpret_cast<const unsigned char *>(W.q16), W.sc, nullptr, part, W.N, M, W.N,
                                W.K, QkvOut(), kps);
+    } else if constexpr (RT == 1 && CT == 5) {
+        // 128 x 320: the plan's, from the f16 copy only, in either block order
+        if (!W.q16) return hipErrorInvalidValue;
+        const unsigned char *q = reinterpret_cast<const unsigned char *>(W.q16);
+        if (gemm_sched() == 1)
+            hipLaunchKernelGGL((k_gemm_lds<EPI_NONE, RT, CT, WM, WN, 0, true, 1>), grid, block, 0, st, Xh, q, W.sc,
+                               nullptr, part, W.N, M, W.N, W.K, QkvOut(), kps);
+        else
+            hipLaunchKernelGGL((k_gemm_lds<EPI_NONE, RT, CT, WM, WN, 0, true>), grid, block, 0, st, Xh, q, W.sc, nullptr,
+                               part, W.N, M, W.N, W.K, QkvOut(), kps);
     } else if (!W.q16 && W.fmt == WF_Q8)
         hipLaunchKernelGGL((k_gemm_lds<EPI_NONE, RT, CT, WM, WN, WF_Q8, true>), grid, block, 0, st, Xh,
                            static_cast<const unsigned char *>(W.q), W.sc, nullptr, part, W.N, M, W.N, W.K, QkvOut(),
@@ -1154,6 +1165,7 @@ hipError_t launch_split(const DevMatrix &W, const void *X, int M, float *part, i
         if (kw == 2) return launch_split_t<1, 2, 2, 2, 2>(W, X, M, part, S, kps, st);
         return launch_split_t<1, 2, 2, 2>(W, X, M, part, S, kps, st);
     }
+    if (tile == LDS_TILE_128x320) return launch_split_t<1, 5, 4, 2>(W, X, M, part, S, kps, st);
     return launch_split_t<2, 2, 2, 2>(W, X, M, part, S, kps, st);
 }
 
@@ -1191,6 +1203,38 @@ int tile_choice(int M, int N, bool copy) {
         }
     }
     return best;
+}
+
+// Tile for an unsplit plain-epilogue GEMM from the f16 copy (or a pair copy:
+// 64-row tiles and 128 x 320 only) by the time its fullest CU takes: n tiles
+// of KB blocks, us, fitted to every tile measured on the ESM-2 35M to 3B
+// projections at 600 to 8192 rows (within 10% of them).  A CU's tiles share
+// its matrix cores, so the 64-row tiles' times add up; 128 x 128 tiles run in
+// pairs; the 8-wave tiles one after the other (128 x 320 over several rounds
+// with plain epilogues as persistent workgroups).  What it corrects: FC1 of
+// 35M at 2729 rows 24.6 -> 20.3 us (64 x 128 instead of 128 x 256), of 150M
+// at 2100 rows 27.4 -> 24.2, of 650M at 700 rows 33.6 -> 29.6.
+int tile_time(int M, int N, int KB, bool pair, int epi) {
+    const long cus = device_cus(), m64 = (M + 63) / 64, m128 = (M + 127) / 128;
+    auto fullest = [&](long mt, int bn) { return (double)((mt * ((N + bn - 1) / bn) + cus - 1) / cus); };
+    const double n64 = fullest(m64, 64), n64x128 = fullest(m64, 128), n128 = fullest(m128, 128),
+                 n256 = fullest(m128, 256), n320 = fullest(m128, 320);
+    const double pairs = (double)((long)n128 / 2), odd = n128 - 2 * pairs;
+    const bool pers = n320 > 1 && !pair && (epi == EPI_GELU_H2 || epi == EPI_NONE);
+    const struct {
+        int tile;
+        double us;
+    } cand[5] = {
+        {LDS_TILE_128x320, n320 * (pers ? 10.0 + 0.92 * KB : 11.6 + 1.02 * KB)},
+        {LDS_TILE_128x256, n256 == 1 ? 12.7 + 0.79 * KB : n256 * (8.9 + 0.87 * KB)},
+        {LDS_TILE_128x128, pairs * (10.0 + 0.89 * KB) + odd * (8.0 + 0.57 * KB)},
+        {LDS_TILE_64x128, n64x128 == 1 ? 5.5 + 0.32 * KB : 4.0 + n64x128 * (1.0 + 0.29 * KB)},
+        {LDS_TILE_64x64, 4.0 + n64 * (0.4 + 0.17 * KB)},
+    };
+    int best = 0;
+    for (int i = 1; i < 5; i++)
+        if (cand[i].us < cand[best].us && !(pair && i < 3)) best = i;
+    return cand[best].tile;
 }
 
 // CIH_GEMM_TILE_N (CIH_GEMM_TILE_N_GELU for the FC1 + GELU GEMM): 320, 256,
@@ -1297,24 +1341,24 @@ hipError_t launch_gemm_lds_split(const DevMatrix &W, const void *X, int M, const
 // Routing of the problems that do not fill the device with 128-row tiles,
 // from a sweep of every tile and split over the ESM-2 8M-3B projections at
 // 16-8192 tokens on MI355X (256 CUs; the thresholds scale with the CU
-// count); below 49 rows k_gemm_rows (49 to 63 rows read a
-// 64-row tile past their end, clamped: as fast as at 64).  One 4-wave workgroup per CU exposes the per-block barrier and
-// operand-read latency to its lone wave per SIMD; smaller tiles put three or
+// count); below 49 rows k_gemm_rows (49 to 63 rows read a 64-row tile past
+// their end, clamped).  One 4-wave workgroup per CU exposes the per-block
+// barrier and operand-read latency to its lone wave per SIMD; smaller tiles put three or
 // four workgroups on each CU and leave fewer CUs idle in the last round.  A
 // split's partial sums cost the LayerNorm that adds them about S M N 4 bytes
 // at 2 TB/s (3B, 2048 x 2560, 3 splits: 10.1 -> 41.6 us), so splits pay only
 // where the unsplit GEMM leaves most of the device idle:
-//   * residual projections with K >= 5120 (160 blocks) whose caller adds
-//     splits, from 25 tiles of 128 x 128 on (fewer: the 64 x 64 rule
-//     below): up to 100 such tiles, 64 x 128 tiles in 3 k-splits;
-//     fewer 128 x 128 tiles than CUs, those in min(2 CUs / tiles, 3)
-//     splits; else the round model's tile, unsplit;
-//   * up to 5 CUs tiles of 64 x 64: that tile, residual projections split
-//     into min(CUs / tiles, 6, blocks / 4) (5 -> 4); when the workgroups
-//     (tiles x splits) leave each CU at most one, two groups of 4 waves share
-//     each tile's k-blocks (below);
-//   * else the round model's large tile (unchanged at the 650M 8192-token
-//     shapes).
+//   * residual projections whose caller adds splits: 128 x 320 tiles in 2 to
+//     4 k-splits where those fill the device (s320 below);
+//   * those with K >= 5120 (160 blocks) from 25 tiles of 128 x 128 on (fewer:
+//     the 64 x 64 rule below): up to 100 such tiles, 64 x 128 tiles in 3
+//     k-splits; fewer 128 x 128 tiles than CUs, those in min(2 CUs / tiles,
+//     3) splits;
+//   * those with at most half as many 64 x 64 tiles as CUs: that tile in
+//     min(CUs / tiles, 6, blocks / 4) splits (5 -> 4);
+//   * else the tile whose fullest CU is done first (tile_time); 64 x 64 tiles
+//     whose workgroups (tiles x splits) leave each CU at most one run on two
+//     groups of 4 waves that share the k-blocks (below).
 // ESM-2 35M at 2552 tokens (8 ragged sequences), against the register-staged
 // kernel and 128 x 160 before: QKV 17.3 -> 14.4, Wo 8.9 -> 8.2, FC1 24.8 ->
 // 20.1, FC2 20.8 -> 21.3 us, and Wo and FC2 no longer leave 3 splits each to
@@ -1333,26 +1377,35 @@ bool gemm_lds_plan(const DevMatrix &W, int a_fmt, int M, int epi, size_t part_fl
     const int KB = W.K / 32;
     const bool can_split = epi == EPI_RESIDUAL && part_floats > 0 && !(ke && !strcmp(ke, "0"));
     int tile, S = 1;
+    // 128 x 320 tiles in 2 to 4 k-splits that fill 80% of the CUs or more, with
+    // 40 blocks or more each (fewer: the fold costs what they gain).  GEMM and
+    // the LayerNorm that adds the splits, us, against the best of the other
+    // tiles and splits: 3B FC2 at 2048 rows 216 against 249 (128 x 256 unsplit,
+    // the choice before: 277), 1024 rows 125 / 134; 650M FC2 at 4096 rows 119 /
+    // 136, 2600 rows 83 / 92, 1616 rows 62 / 68; 3B Wo at 2048 rows 77 / 81.
+    // Below 80%: 3B FC2 at 1500 rows (192 workgroups) 194 / 178.
+    const long t320 = (long)((M + 127) / 128) * ((W.N + 319) / 320);
+    int s320 = can_split && !W.kx ? (int)std::min<long>(cus / t320, 4) : 1;
+    if (s320 >= 2 && (t320 * s320 * 10 < cus * 8 || KB / s320 < 40)) s320 = 1;
     if (const int forced = tile_env(epi)) {
         tile = forced;
-    } else if (can_split && KB >= 160 && t128 * 256 > 25 * cus) {
+    } else if (s320 >= 2) {
+        tile = LDS_TILE_128x320;
+        S = s320;
+    } else if (can_split && KB >= 160 && t128 * 256 > 25 * cus && t128 < cus) {
         if (t128 * 256 <= 100 * cus) {
             tile = LDS_TILE_64x128;
             S = 3;
-        } else if (t128 < cus) {
+        } else {
             tile = LDS_TILE_128x128;
             S = (int)std::min<long>(2 * cus / t128, 3);
-        } else {
-            tile = tile_choice(M, W.N, true);
         }
-    } else if (t64 <= 5 * cus) {
+    } else if (can_split && 2 * t64 <= cus) {
         tile = LDS_TILE_64x64;
-        if (can_split) {
-            S = (int)std::max<long>(1, std::min<long>({cus / t64, 6, KB / 4}));
-            if (S == 5) S = 4;
-        }
+        S = (int)std::max<long>(1, std::min<long>({cus / t64, 6, KB / 4}));
+        if (S == 5) S = 4;
     } else {
-        tile = tile_choice(M, W.N, true);
+        tile = tile_time(M, W.N, KB, W.kx != 0, epi);
     }
     // a pair copy (W.kx): the 64-row tiles and 128 x 320 (the others keep the
     // register-staged pair path)

@@ -265,3 +265,31 @@ def test_lm_head_limb_handoff_is_bit_identical(case, monkeypatch):
         n = len(s)
         assert np.array_equal(a["logits"][i, :n], b["logits"][i, :n]), (case, i)
         assert np.array_equal(c["logits"][i, :n], b["logits"][i, :n]), (case, i)
+
+
+@pytest.mark.parametrize("d,F,H,lens", [
+    (640, 2560, 20, [511] * 12 + [397]),   # FC2 on 128 x 320 tiles in 2 splits (52 x 2 tiles, a partial last row tile)
+    (1280, 5120, 20, [517, 513, 510]),     # FC2 in 4 splits of 40 blocks
+    (1280, 5120, 20, [520] * 5),           # FC2 in 3 splits, the last shorter
+    (480, 1920, 20, [512, 131, 387, 254, 449, 173, 318, 505]),  # FC1 on 64 x 128 tiles past 1280 tiles of 64 x 64
+    (640, 2560, 20, [700, 700, 701])])
+@pytest.mark.parametrize("dtype", [1, 2])
+def test_plan_matches_the_routes_without_it(d, F, H, lens, dtype, monkeypatch):
+    """Tiles and splits of the plan against the routes without it (CIH_GEMM_PLAN=0): the same products summed in
+    another order where K is split, 1e-5 of the largest value."""
+    cfg = ch.EsmConfig(d, F, 1, H)
+    w = ch.EsmWeights.random(cfg, seed=d, std=0.03, bias_std=0.02)
+    w = w.quantize_q8() if dtype == 1 else w.quantize_q4()
+    rng = np.random.default_rng(F)
+    seqs = [np.concatenate([[0], 4 + rng.integers(0, 20, n - 2), [2]]).astype(np.int32) for n in lens]
+    flags = ch.OUT_LOGITS | ch.OUT_HIDDEN
+    got = []
+    for env in (None, "0"):
+        if env:
+            monkeypatch.setenv("CIH_GEMM_PLAN", env)
+        m = ch.GpuModel(cfg, w, max_batch=len(seqs), max_len=max(lens), outputs=flags)
+        got.append(m.forward(seqs, flags))
+        m.close()
+    for k in ("logits", "hidden"):
+        assert np.isfinite(got[0][k]).all()
+        assert np.abs(got[0][k] - got[1][k]).max() <= 1e-5 * max(1.0, np.abs(got[1][k]).max()), k
