@@ -45,6 +45,13 @@ __global__ __launch_bounds__(DEC_THREADS) void k_rope_kv(float *__restrict__ qkv
 
 constexpr int ATT_THREADS = 512;  // 8 waves per (row, head)
 
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+// v of the lane that DPP control C names (all lanes read a valid one)
+template <int C> __device__ __forceinline__ float dpp(float v) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), C, 0xf, 0xf, true));
+}
+
 __device__ __forceinline__ float block_reduce(float v, float *scratch, bool is_max) {
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) {
@@ -62,10 +69,18 @@ __device__ __forceinline__ float block_reduce(float v, float *scratch, bool is_m
 }
 
 // One workgroup per (row, head).  Scores s_t = (q . k_t) / sqrt(hd) for
-// t = 0..pos (a thread per key), softmax as softmax() (lib.rs:3500-3504:
-// max, exp(s - max), 1 / sum), then out = sum_t p_t v_t with G = 512 / HD
-// key groups of HD lanes (a group reads whole V rows, four rows in flight)
-// whose partial sums are added in group order.
+// t = 0..pos, softmax as softmax() (lib.rs:3500-3504: max, exp(s - max),
+// 1 / sum), then out = sum_t p_t v_t.  Bound by reading the slot's K and V
+// (512 bytes a key at hd 64) at the 45 B/ns a CU takes: L = HD / 4 lanes read
+// a row in 16-byte pieces, so a wave's load covers 64 / L whole rows, and
+// each wave has U such loads in flight, the first U of K and of V requested
+// before anything else.  A key's score is added over its lanes, an output
+// dim over a lane's keys, the wave's key groups and the waves, in that order.
+// (A thread per key row, and V rows four at a time by 64 lanes, took 28.8 us
+// per layer for 8 rows at position 700 of 650M and 13.9 us for one at 280;
+// now 17.4 and 10.6; a prompt's rows 97 -> 61 us at 256 rows per call.
+// Keeping V's second sweep in K's registers under the softmax changed neither
+// and cost the prompt's rows their second workgroup per CU, 61 -> 101.)
 //
 // FUSED (each slot at most once in the launch): the workgroup also applies
 // RoPE to its head's Q and K, writes K and V at pos into the cache for later
@@ -91,12 +106,14 @@ __global__ __launch_bounds__(ATT_THREADS) void k_decode_attention(const float *_
                                                                   const unsigned char *__restrict__ wo_q = nullptr,
                                                                   const float *__restrict__ wo_sc = nullptr,
                                                                   int wo_n = 0) {
-    constexpr int G = ATT_THREADS / HD;
-    constexpr int HALF = HD / 2;
-    extern __shared__ float sm[];
+    constexpr int HALF = HD / 2, NWV = ATT_THREADS / 64;
+    constexpr int LK = HD == 24 ? 8 : HD / 4;  // lanes per key (hd 24: lanes 6 and 7 of 8 idle)
+    constexpr int KW = 64 / LK, U = 8;         // keys per load of a wave, loads in flight
+    constexpr int STEP = NWV * KW * U;         // keys per sweep of the workgroup
+    extern __shared__ __attribute__((aligned(16))) float sm[];
     float *qs = sm;                        // [HD] rotated query
     float *kcur = qs + HD, *vcur = kcur + HD;  // [HD] key and value at pos (FUSED)
-    float *gsum = vcur + HD;               // [G][HD] per-group partial outputs
+    float *gsum = vcur + HD;               // [NWV][HD] per-wave partial outputs
     float *red = gsum + ATT_THREADS;       // [8]
     float *p = red + 8;                    // [pos + 1]
     const int r = blockIdx.x, h = blockIdx.y;
@@ -110,21 +127,24 @@ __global__ __launch_bounds__(ATT_THREADS) void k_decode_attention(const float *_
     const int wc0 = (int)blockIdx.z * 128 * WP, wc1 = min(wc0 + 128 * WP, wo_n);
     if constexpr (WOF != 0) wo.load(wo_q, wo_sc, wo_n, h * NKB, NKB, wc0, wc1);
     const bool cache_writer = WOF == 0 || blockIdx.z == 0;
-    // This thread's first key row is requested before anything waits, so its
-    // latency overlaps the gather, the rotation and the barriers.
-    float4 kfirst[HD / 4];
-    if (t < n_cached) {
-        const float4 *kr = reinterpret_cast<const float4 *>(K + (size_t)t * d);
+    // key j of (sweep s0, load u): s0 + (u NWV + wave) KW + lane / LK; this
+    // lane's quad of its dims
+    const int lane = t & 63, wave = t >> 6, kq = lane / LK, dl = 4 * min(lane % LK, HD / 4 - 1);
+    const bool live = lane % LK < HD / 4;
+    const float *Kl = K + dl, *Vl = V + dl;
+    auto key = [&](int s0, int u) __attribute__((always_inline)) { return s0 + (u * NWV + wave) * KW + kq; };
+    // keys past the cached ones re-read the last (their scores are not stored, their weights zero)
+    auto fetch = [&](const float *base, int s0, f32x4 (&v)[U]) __attribute__((always_inline)) {
 #pragma unroll
-        for (int i = 0; i < HD / 4; i++) kfirst[i] = kr[i];
-    }
-    // likewise the first four V rows of this lane's group (P.V below)
-    const int g = t / HD, i = t - g * HD;
-    float vfirst[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-    if (g < G) {
-#pragma unroll
-        for (int u = 0; u < 4; u++)
-            if (g + u * G < n_cached) vfirst[u] = V[(size_t)(g + u * G) * d + i];
+        for (int u = 0; u < U; u++)
+            v[u] = *reinterpret_cast<const f32x4 *>(base + (size_t)min(key(s0, u), n_cached - 1) * d);
+    };
+    // The first sweep of K and of V is requested before anything waits, so its
+    // latency overlaps the gather, the rotation, the softmax and the barriers.
+    f32x4 kv[U], vv[U];
+    if (n_cached > 0) {
+        fetch(Kl, 0, kv);
+        fetch(Vl, 0, vv);
     }
     if constexpr (FUSED) {
         float c = 0.0f, s = 0.0f;
@@ -175,34 +195,33 @@ __global__ __launch_bounds__(ATT_THREADS) void k_decode_attention(const float *_
         if (t < HD) qs[t] = q[t];
     }
     __syncthreads();
-    float mx = -INFINITY;
-    for (int j = t; j <= pos; j += ATT_THREADS) {
-        float acc = 0.0f;
-        if (j < n_cached) {
-            float4 kv4[HD / 4];
-            if (j == t) {
+    const f32x4 q4 = *reinterpret_cast<const f32x4 *>(qs + dl);
+    // a key's products over its lanes: DPP adds within 16 lanes (quads, halves
+    // of 8, mirrored: partners hold equal sums by then)
+    auto key_sum = [&](f32x4 k) __attribute__((always_inline)) {
+        float a = live ? fmaf(q4.w, k.w, fmaf(q4.z, k.z, fmaf(q4.y, k.y, q4.x * k.x))) : 0.0f;
+        a += dpp<0xB1>(a);                            // lane ^ 1
+        a += dpp<0x4E>(a);                            // lane ^ 2
+        if constexpr (LK >= 8) a += dpp<0x141>(a);    // mirrored in 8
+        if constexpr (LK >= 16) a += dpp<0x140>(a);   // mirrored in 16
+        return a;
+    };
+    for (int s0 = 0; s0 < n_cached; s0 += STEP) {
+        float a[U];
 #pragma unroll
-                for (int i = 0; i < HD / 4; i++) kv4[i] = kfirst[i];
-            } else {
-                const float4 *kr = reinterpret_cast<const float4 *>(K + (size_t)j * d);
+        for (int u = 0; u < U; u++) a[u] = key_sum(kv[u]);
+        if (s0 + STEP < n_cached) fetch(Kl, s0 + STEP, kv);
 #pragma unroll
-                for (int i = 0; i < HD / 4; i++) kv4[i] = kr[i];
-            }
-#pragma unroll
-            for (int i = 0; i < HD / 4; i++) {
-                acc = fmaf(qs[4 * i], kv4[i].x, acc);
-                acc = fmaf(qs[4 * i + 1], kv4[i].y, acc);
-                acc = fmaf(qs[4 * i + 2], kv4[i].z, acc);
-                acc = fmaf(qs[4 * i + 3], kv4[i].w, acc);
-            }
-        } else {
-#pragma unroll
-            for (int i = 0; i < HD; i++) acc = fmaf(qs[i], kcur[i], acc);
-        }
-        const float sc = acc * inv_scale;
-        p[j] = sc;
-        mx = fmaxf(mx, sc);
+        for (int u = 0; u < U; u++)
+            if (lane % LK == 0 && key(s0, u) < n_cached) p[key(s0, u)] = a[u] * inv_scale;
     }
+    if (FUSED && wave == 0) {
+        const float a = key_sum(*reinterpret_cast<const f32x4 *>(kcur + dl));
+        if (lane == 0) p[pos] = a * inv_scale;
+    }
+    __syncthreads();
+    float mx = -INFINITY;
+    for (int j = t; j <= pos; j += ATT_THREADS) mx = fmaxf(mx, p[j]);
     mx = block_reduce(mx, red, true);
     float sum = 0.0f;
     for (int j = t; j <= pos; j += ATT_THREADS) {
@@ -213,32 +232,34 @@ __global__ __launch_bounds__(ATT_THREADS) void k_decode_attention(const float *_
     sum = block_reduce(sum, red, false);
     const float inv = 1.0f / sum;
     __syncthreads();
-    if (g < G) {
-        const float *vi = V + i;
-        float a0 = 0.0f, a1 = 0.0f, a2 = 0.0f, a3 = 0.0f;
-        // rows g, g+G, g+2G, g+3G from the registers, then four at a time
-        if (g < n_cached) a0 = p[g] * inv * vfirst[0];
-        if (g + G < n_cached) a1 = p[g + G] * inv * vfirst[1];
-        if (g + 2 * G < n_cached) a2 = p[g + 2 * G] * inv * vfirst[2];
-        if (g + 3 * G < n_cached) a3 = p[g + 3 * G] * inv * vfirst[3];
-        int j = g + 4 * G;
-        for (; j + 3 * G < n_cached; j += 4 * G) {
-            const float v0 = vi[(size_t)j * d], v1 = vi[(size_t)(j + G) * d];
-            const float v2 = vi[(size_t)(j + 2 * G) * d], v3 = vi[(size_t)(j + 3 * G) * d];
-            a0 = fmaf(p[j] * inv, v0, a0);
-            a1 = fmaf(p[j + G] * inv, v1, a1);
-            a2 = fmaf(p[j + 2 * G] * inv, v2, a2);
-            a3 = fmaf(p[j + 3 * G] * inv, v3, a3);
+    f32x4 o4 = {0.0f, 0.0f, 0.0f, 0.0f};
+    for (int s0 = 0; s0 < n_cached; s0 += STEP) {
+        if (s0 > 0) fetch(Vl, s0, vv);
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const int j = key(s0, u);
+            const float w = j < n_cached ? p[j] * inv : 0.0f;
+#pragma unroll
+            for (int e = 0; e < 4; e++) o4[e] = fmaf(w, vv[u][e], o4[e]);
         }
-        for (; j < n_cached; j += G) a0 = fmaf(p[j] * inv, vi[(size_t)j * d], a0);
-        if (FUSED && pos >= g && (pos - g) % G == 0) a0 = fmaf(p[pos] * inv, vcur[i], a0);
-        gsum[g * HD + i] = (a0 + a1) + (a2 + a3);
     }
+    if (FUSED && wave == 0 && kq == 0) {
+        const float w = p[pos] * inv;
+        const f32x4 v = *reinterpret_cast<const f32x4 *>(vcur + dl);
+#pragma unroll
+        for (int e = 0; e < 4; e++) o4[e] = fmaf(w, v[e], o4[e]);
+    }
+    // the wave's key groups, then the waves
+#pragma unroll
+    for (int o = LK; o < 64; o <<= 1)
+#pragma unroll
+        for (int e = 0; e < 4; e++) o4[e] += __shfl_xor(o4[e], o);
+    if (kq == 0 && live) *reinterpret_cast<f32x4 *>(gsum + wave * HD + dl) = o4;
     __syncthreads();
     if (t < HD) {
         float o = gsum[t];
 #pragma unroll
-        for (int k = 1; k < G; k++) o += gsum[k * HD + t];
+        for (int k = 1; k < NWV; k++) o += gsum[k * HD + t];
         if constexpr (WOF != 0) qs[t] = o;  // the query is no longer read
         else if constexpr (OF == AF_H2) h2_store(reinterpret_cast<unsigned short *>(out), r, h * HD + t, d, o);
         else out[(size_t)r * d + h * HD + t] = o;
