@@ -130,8 +130,7 @@ __global__ __launch_bounds__(256) void k_rln4(float *__restrict__ x, const float
 #pragma unroll
     for (int i = 0; i < PER; i++)
         if (lane + 64 * i < n4) s += (v[i].x + v[i].y) + (v[i].z + v[i].w);
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o);
+    s = wave_butterfly(s);
     const float mean = s / (float)d;
     float q = 0.0f;
 #pragma unroll
@@ -139,8 +138,7 @@ __global__ __launch_bounds__(256) void k_rln4(float *__restrict__ x, const float
         const f32x4 t = v[i] - mean;
         if (lane + 64 * i < n4) q += (t.x * t.x + t.y * t.y) + (t.z * t.z + t.w * t.w);
     }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) q += __shfl_xor(q, o);
+    q = wave_butterfly(q);
     const float var = q / (float)d;
     const float inv = 1.0f / sqrtf(var + 1e-5f);
     if (flag && lane == 0 && !(__builtin_isfinite(mean) && __builtin_isfinite(var))) atomicOr(flag, FLAG_NONFINITE);

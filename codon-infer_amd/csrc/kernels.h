@@ -78,6 +78,34 @@ __device__ __forceinline__ float fold_splits(const float *__restrict__ p, int S,
     return acc;
 }
 typedef float fold4_t __attribute__((ext_vector_type(4)));
+// Sum of v over the wave, the same in every lane: the butterfly over lanes
+// ^ 32, 16, 8, 4, 2, 1 without LDS round trips (permlane swaps and DPP; each
+// step adds the same two values as a __shfl_xor step, so the same bits).  A
+// row's two sums were 12 dependent LDS trips: k_rln of 8 rows 5.2 -> 4.7 us,
+// k_layernorm4 of 8192 x 1280 16.1 -> 15.2.
+template <int C, int BANK> __device__ __forceinline__ float dpp_or(float old, float v) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(__builtin_bit_cast(int, old), __builtin_bit_cast(int, v),
+                                                                 C, 0xf, BANK, false));
+}
+__device__ __forceinline__ float wave_butterfly(float v) {
+    // the swaps exchange lane halves between two registers: w is v in a
+    // register of its own (given one value twice, the compiler uses one)
+    float w = v;
+    asm volatile("" : "+v"(w));
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(w), false, false);
+    const unsigned r0 = r[0], r1 = r[1];
+    v = __uint_as_float(r0) + __uint_as_float(r1);
+    w = v;
+    asm volatile("" : "+v"(w));
+    const auto t = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(w), false, false);
+    const unsigned t0 = t[0], t1 = t[1];
+    v = __uint_as_float(t0) + __uint_as_float(t1);
+    v += dpp_or<0x128, 0xf>(v, v);                               // ^ 8: rotation by 8 of 16
+    v += dpp_or<0x114, 0xa>(dpp_or<0x104, 0x5>(v, v), v);        // ^ 4: shifts by 4 of the even and odd quads
+    v += dpp_or<0x4E, 0xf>(v, v);                                // ^ 2
+    v += dpp_or<0xB1, 0xf>(v, v);                                // ^ 1
+    return v;
+}
 // Mean and variance of one row of n4 quads held in LDS, formed by one wave:
 // lane l sums quads l, l + 64, ... in order, then a butterfly (the
 // reduction order of k_layernorm4, shared by every kernel that normalises a
@@ -85,16 +113,14 @@ typedef float fold4_t __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ void row_stats64(const fold4_t *xs, int n4, int d, int lane, float &mean, float &var) {
     float s = 0.0f;
     for (int c = lane; c < n4; c += 64) s += (xs[c].x + xs[c].y) + (xs[c].z + xs[c].w);
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o);
+    s = wave_butterfly(s);
     mean = s / (float)d;
     float q = 0.0f;
     for (int c = lane; c < n4; c += 64) {
         const fold4_t t = xs[c] - mean;
         q += (t.x * t.x + t.y * t.y) + (t.z * t.z + t.w * t.w);
     }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) q += __shfl_xor(q, o);
+    q = wave_butterfly(q);
     var = q / (float)d;
 }
 // (CH loads in flight at a time: fewer registers for kernels that fold many

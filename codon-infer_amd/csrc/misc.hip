@@ -6,11 +6,7 @@
 
 namespace cih {
 
-__device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
-    return v;
-}
+__device__ __forceinline__ float wave_sum(float v) { return wave_butterfly(v); }
 
 // Embedding + token-dropout rescale (codon-infer src/lib.rs:5117-5131; Q8
 // 5461-5479; Q4 5820-5833).  scale = 0.88 / (1 - mask_count/len) for the
