@@ -1668,7 +1668,17 @@ hipError_t launch_attention(const float *qkv, int d, int H, SeqMeta sm, const fl
     // waves of each 32-query task split its keys instead (k_attention_xs);
     // the switches of the key split turn it off.
     const int nq32 = (sm.S_max + 31) / 32, t32 = sm.B * H * nq32;
-    const bool xsplit = !fp32 && attention_wave_split(sm.B, sm.S_max, H);
+    // Up to three tasks per CU it also pays on 4 waves, for sequences of at
+    // most 16 tiles and head sizes up to 32 (three workgroups fit a CU's LDS;
+    // no merge kernel) or with an export (no key split otherwise): 150M FP32
+    // B=3 (347, 61, 190) 2.76 -> 2.62 ms per forward, 150M Q8_0 B=3 2.49 -> 2.28,
+    // 8M FP32 B=3 with maps 0.405 -> 0.361, 650M Q8_0 B=2 (500, 300) with
+    // contacts 6.57 -> 6.37.  Not beyond: 35M B=4 (880 tasks) 0.804 -> 0.819,
+    // 150M L=900 (29 tiles) 2.69 -> 2.74, 650M L=402 without an export 3.67 ->
+    // 3.84.
+    const bool split_on = !(se && !strcmp(se, "0")) && !(ke && !strcmp(ke, "0"));
+    const bool xs4 = split_on && !qe && (hd <= 32 || P) && t32 <= 3 * device_cus() && nq32 <= 16;
+    const bool xsplit = !fp32 && (attention_wave_split(sm.B, sm.S_max, H) || xs4);
 #define CIH_ATT_K(KER, HDV, ONE)                                                                                \
     hipLaunchKernelGGL((KER<HDV, ONE>), dim3((sm.S_max + 127) / 128, H, sm.B), dim3(256), 0, st, qkv, d, sm.cu, \
                        sm.lens, sm.S_max, rope_cos, rope_sin, out, out_fmt, P, (long long)pb, (long long)ph,     \
@@ -1684,7 +1694,7 @@ hipError_t launch_attention(const float *qkv, int d, int H, SeqMeta sm, const fl
 #define CIH_ATT_XS(HDV, MODE)                                                                                   \
     do {                                                                                                        \
         if (nq32 <= 2) CIH_ATT_XSK(HDV, 2, MODE);                                                               \
-        else if (nq32 <= 4) CIH_ATT_XSK(HDV, 4, MODE);                                                          \
+        else if (nq32 <= 4 || t32 > device_cus()) CIH_ATT_XSK(HDV, 4, MODE);                                    \
         else CIH_ATT_XSK(HDV, 8, MODE);                                                                         \
     } while (0)
 #define CIH_ATT(HDV)                                                                                           \

@@ -706,3 +706,25 @@ def test_graph_key_follows_kernel_switches(monkeypatch):
     diff = float(np.abs(a["hidden"] - b["hidden"]).max())
     assert 0.0 < diff <= 1e-3, diff
     assert np.array_equal(a["hidden"], c["hidden"]) and np.array_equal(a["logits"], c["logits"])
+
+
+@pytest.mark.parametrize("flags", [ch.OUT_LOGITS, ch.OUT_LOGITS | ch.OUT_ATTN])
+@pytest.mark.parametrize("hd,H", [(16, 20), (24, 20), (32, 20), (64, 10)])
+@pytest.mark.parametrize("lens", [[290, 33, 161], [512, 97]])
+def test_attention_four_wave_split(lens, hd, H, flags, monkeypatch):
+    """Batches of one to three 32-query tasks per CU, whose tasks run on 4 waves (up to 16 key tiles, four per wave):
+    against the oracle, and against the route without the split (CIH_ATT_SPLIT=0), 1e-5 as FP32 sums regrouped."""
+    cfg = ch.EsmConfig(hd * H, 320, 2, H)
+    w = ch.EsmWeights.random(cfg, seed=hd, std=0.05, bias_std=0.02)
+    rng = np.random.default_rng(hd)
+    seqs = [rand_tokens(rng, n - 2) for n in lens]
+    check_batch(cfg, w, seqs, flags)
+    got = []
+    for env in (None, "0"):
+        if env:
+            monkeypatch.setenv("CIH_ATT_SPLIT", env)
+        m = ch.GpuModel(cfg, w, max_batch=len(seqs), max_len=max(lens), outputs=flags)
+        got.append(m.forward(seqs, flags))
+        m.close()
+    for k in [k for k in got[0] if k != "lens"]:
+        assert np.abs(got[0][k] - got[1][k]).max() <= 1e-5 * max(1.0, np.abs(got[1][k]).max()), k
