@@ -293,8 +293,8 @@ int cih_model_reserve(cih_model *m, int32_t max_batch, int32_t max_seq_len, uint
     }
     if (good && (flags & CIH_OUT_CONTACTS))
         good = ok(dalloc(ws.M, B * n * n, dl)) && ok(dalloc(ws.r, L * H * B * n, dl)) &&
-               ok(dalloc(ws.coef, L * H * B, dl)) && ok(dalloc(ws.rowsum, B * H * S, dl)) &&
-               ok(dalloc(ws.colpart, apc_colpart_floats((int)B, (int)H, (int)n), dl));
+               ok(dalloc(ws.coef, L * H * B, dl)) && ok(dalloc(ws.rowsum, L * B * H * S, dl)) &&
+               ok(dalloc(ws.colpart, apc_colpart_floats((int)B, std::max(m->n_lhs, 1), (int)n), dl));
     if (good && !(flags & CIH_IO_DEVICE)) {
         if (flags & CIH_OUT_LOGITS) good = good && ok(dalloc(ws.o_logits, T * V, dl));
         if (flags & CIH_OUT_HIDDEN) good = good && ok(dalloc(ws.o_hidden, T * d, dl));
@@ -482,8 +482,10 @@ int forward_impl(cih_model *m, const int32_t *tokens, const int32_t *lens, int32
         HIPCHK(launch_kv_setup(sm, (int)m->hd, H, ws.kv_tb, ws.kv_pk, ws.kv_pos, ws.kv_ti, ws.kv_img, st));
     }
 
-    for (int l = 0; l < L; l++) {
+    for (int l = 0, lh = 0; l < L; l++) {
         const Layer &ly = m->layers[l];
+        const int lh0 = lh;  // this layer's first layer-head of nonzero contact weight
+        lh += m->nz[l];
         // probabilities: straight into the attention-map output when exported
         float *P = nullptr;
         int64_t pb = 0, ph = SS;
@@ -534,14 +536,14 @@ int forward_impl(cih_model *m, const int32_t *tokens, const int32_t *lens, int32
                 double fl = 0;
                 for (int b = 0; b < B; b++) fl += 4.0 * (double)lens[b] * lens[b] * d;
                 ProfScope ps(m, CIH_KC_ATTENTION, fl, 16.0 * T * d);
-                float *rsum = want_contacts && m->nz[l] > 0 ? ws.rowsum : nullptr;
+                float *rsum = want_contacts && m->nz[l] > 0 ? ws.rowsum + (size_t)l * B * H * S_max : nullptr;
                 HIPCHK(launch_attention(ws.qkv, d, H, sm, ws.rope_c, ws.rope_s, ws.ao, af, P, pb, ph, rsum, ws.attp,
                                         ws.attp_floats, st, order, m->nz[l]));
             }
             if (want_contacts && m->nz[l] > 0) {
                 ProfScope ps(m, CIH_KC_OTHER, 0, 0);
-                HIPCHK(launch_apc_layer(P, pb, ph, H, l, m->d_contact_w, m->d_heads + (size_t)l * H, m->nz[l], sm,
-                                        ws.rowsum, ws.colpart, ws.M, ws.r, st));
+                HIPCHK(launch_apc_layer(P, pb, ph, H, l, m->d_contact_w, m->d_heads + (size_t)l * H, m->nz[l],
+                                        lh0, sm, ws.colpart, ws.M, st));
             }
             if (want_final && l == L - 1) {
                 ProfScope ps(m, CIH_KC_OTHER, 0, 0);
@@ -601,7 +603,7 @@ int forward_impl(cih_model *m, const int32_t *tokens, const int32_t *lens, int32
             double fl = 0;
             for (int b = 0; b < B; b++) fl += 4.0 * (double)lens[b] * lens[b] * d;
             ProfScope ps(m, CIH_KC_ATTENTION, fl, 16.0 * T * d);
-            float *rsum = want_contacts && m->nz[l] > 0 ? ws.rowsum : nullptr;
+            float *rsum = want_contacts && m->nz[l] > 0 ? ws.rowsum + (size_t)l * B * H * S_max : nullptr;
             if (use_img)
                 HIPCHK(launch_attention_img(ws.qkv, d, H, sm, ws.kv_tb, ws.kv_img, ws.rope_c, ws.rope_s, ws.ao, af, P,
                                             pb, ph, rsum, ws.attp, ws.attp_floats, st, order, m->nz[l]));
@@ -611,8 +613,8 @@ int forward_impl(cih_model *m, const int32_t *tokens, const int32_t *lens, int32
         }
         if (want_contacts && m->nz[l] > 0) {
             ProfScope ps(m, CIH_KC_OTHER, 0, 0);
-            HIPCHK(launch_apc_layer(P, pb, ph, H, l, m->d_contact_w, m->d_heads + (size_t)l * H, m->nz[l], sm,
-                                    ws.rowsum, ws.colpart, ws.M, ws.r, st));
+            HIPCHK(launch_apc_layer(P, pb, ph, H, l, m->d_contact_w, m->d_heads + (size_t)l * H, m->nz[l],
+                                    lh0, sm, ws.colpart, ws.M, st));
         }
         if (want_final && l == L - 1) {
             ProfScope ps(m, CIH_KC_OTHER, 0, 0);
@@ -639,8 +641,8 @@ int forward_impl(cih_model *m, const int32_t *tokens, const int32_t *lens, int32
     }
     if (want_contacts) {
         ProfScope ps(m, CIH_KC_OTHER, 0, 0);
-        HIPCHK(launch_apc_finalize(ws.M, ws.r, ws.coef, m->d_contact_w, m->d_lhs, m->n_lhs, sm, m->contact_b,
-                                   t_contacts, n_max, st));
+        HIPCHK(launch_apc_finalize(ws.M, ws.rowsum, ws.colpart, ws.r, ws.coef, m->d_contact_w, m->d_lhs, m->n_lhs, H,
+                                   sm, m->contact_b, t_contacts, n_max, st));
     }
     // final LayerNorm: state.x = LN_f(x) (lib.rs:5379-5387).  It also
     // reports a residual row that is no longer finite (the f16 limbs hold

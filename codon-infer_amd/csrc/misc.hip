@@ -272,8 +272,10 @@ hipError_t launch_head_mean(const float *P, int64_t pb, int64_t ph, int H, SeqMe
 // Summed over heads: logit = M + M^T - sum_h (w_h / T_h) r_h r_h^T with
 // M = sum_h w_h A_h, and r_i = (row sum of A)_i + (column sum of A)_i.  The
 // attention kernel supplies the row sums; k_apc_tile reads each map once,
-// accumulating M and column partial sums of `rows` map rows, which k_apc_r
-// adds in order.  M: [B][n_max][n_max], r: [L*H][B][n_max], n_max = S_max - 2.
+// accumulating M and column partial sums of `rows` map rows; one k_apc_r after
+// the last layer adds those of every layer-head in order (a launch per layer
+// was 4.8 us each: 4% of a 650M L=257 forward).  M: [B][n_max][n_max], r:
+// [n_lhs][B][n_max] over the layer-heads of nonzero weight, n_max = S_max - 2.
 constexpr int APC_HMAX = 40;     // most heads of any preset (3B)
 constexpr int APC_ROWS_MIN = 8;  // map rows per wave of k_apc_tile: 8, 16 or 32
 
@@ -291,8 +293,8 @@ static int apc_rows(int B, int n_max) {
 // Enough for every call of at most B sequences and n_max residues: whole
 // 32-row tiles, or, where the rows were halved, fewer than 2 x 8 waves per CU
 // of 64 columns each.
-size_t apc_colpart_floats(int B, int H, int n_max) {
-    return (size_t)H * std::max((size_t)B * ((n_max + 31) / 32) * n_max, (size_t)2 * 8 * device_cus() * 64);
+size_t apc_colpart_floats(int B, int n_lhs, int n_max) {
+    return (size_t)n_lhs * std::max((size_t)B * ((n_max + 31) / 32) * n_max, (size_t)2 * 8 * device_cus() * 64);
 }
 
 // One wave = 64 residue columns x `rows` map rows.  HM >= nz heads per pass
@@ -304,7 +306,7 @@ size_t apc_colpart_floats(int B, int H, int n_max) {
 template <int HM, int R>
 __global__ __launch_bounds__(64) void k_apc_tile(const float *__restrict__ P, long long pb, long long ph, int H,
                                                  int l, const float *__restrict__ w, const int *__restrict__ heads,
-                                                 int nz, const int *__restrict__ lens, int S_max, int rows,
+                                                 int nz, int lh0, const int *__restrict__ lens, int S_max, int rows,
                                                  float *__restrict__ M, float *__restrict__ colpart, int B) {
     const int tile = blockIdx.x, b = blockIdx.z;
     const int n = lens[b] - 2, n_max = S_max - 2, ntiles = (n_max + rows - 1) / rows;
@@ -356,22 +358,21 @@ __global__ __launch_bounds__(64) void k_apc_tile(const float *__restrict__ P, lo
     }
 #pragma unroll
     for (int k = 0; k < HM; k++)
-        if (k < nz) colpart[(((size_t)b * nz + k) * ntiles + tile) * n_max + j] = cs[k];
+        if (k < nz) colpart[(((size_t)(lh0 + k) * B + b) * ntiles + tile) * n_max + j] = cs[k];
 }
 
-// r[l*H + h][b][i] = rowsum[b][h][i+1] + column partials of i in tile order,
-// four waves of every fourth group of 8 tiles (8 loads in flight each) joined
-// in wave order
+// r[k][b][i] of layer-head lhs[k] = l H + h: rowsum[l][b][h][i+1] + column
+// partials of i in tile order, four waves of every fourth group of 8 tiles (8
+// loads in flight each) joined in wave order
 __global__ __launch_bounds__(256) void k_apc_r(const float *__restrict__ rowsum, const float *__restrict__ colpart,
-                                               int H, int l, const int *__restrict__ heads, int nz,
-                                               const int *__restrict__ lens, int S_max, int rows,
-                                               float *__restrict__ r, int B) {
-    const int b = blockIdx.z, k = blockIdx.y, h = heads[k];
+                                               int H, const int *__restrict__ lhs, const int *__restrict__ lens,
+                                               int S_max, int rows, float *__restrict__ r, int B) {
+    const int b = blockIdx.z, k = blockIdx.y, l = lhs[k] / H, h = lhs[k] % H;
     const int n = lens[b] - 2, n_max = S_max - 2, ntiles = (n_max + rows - 1) / rows;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, i = blockIdx.x * 64 + lane;
     __shared__ float part[3][64];
     const int nt = n > 0 ? (n + rows - 1) / rows : 0;
-    const float *cp = colpart + ((size_t)b * nz + k) * ntiles * n_max + i;
+    const float *cp = colpart + ((size_t)k * B + b) * ntiles * n_max + i;
     float c = 0.0f;
     if (i < n)
         for (int t0 = wave * 8; t0 < nt; t0 += 32) {
@@ -386,19 +387,19 @@ __global__ __launch_bounds__(256) void k_apc_r(const float *__restrict__ rowsum,
     __syncthreads();
     if (wave || i >= n) return;
     c = ((c + part[0][lane]) + part[1][lane]) + part[2][lane];
-    r[((size_t)(l * H + h) * B + b) * n_max + i] = rowsum[((size_t)b * H + h) * S_max + i + 1] + c;
+    r[((size_t)k * B + b) * n_max + i] = rowsum[(((size_t)l * B + b) * H + h) * S_max + i + 1] + c;
 }
 
 hipError_t launch_apc_layer(const float *P, int64_t pb, int64_t ph, int H, int l, const float *w_dev,
-                            const int *heads_dev, int n_heads_nz, SeqMeta sm, const float *rowsum, float *colpart,
-                            float *M, float *r, hipStream_t st) {
+                            const int *heads_dev, int n_heads_nz, int lh0, SeqMeta sm, float *colpart, float *M,
+                            hipStream_t st) {
     if (n_heads_nz <= 0 || sm.S_max < 3) return hipSuccess;
     if (n_heads_nz > APC_HMAX || H > APC_HMAX) return hipErrorInvalidValue;
     const int n_max = sm.S_max - 2, rows = apc_rows(sm.B, n_max);
     const dim3 tg((n_max + rows - 1) / rows, (n_max + 63) / 64, sm.B);
 #define CIH_APC(HM, R)                                                                                              \
     hipLaunchKernelGGL((k_apc_tile<HM, R>), tg, dim3(64), 0, st, P, (long long)pb, (long long)ph, H, l, w_dev,       \
-                       heads_dev, n_heads_nz, sm.lens, sm.S_max, rows, M, colpart, sm.B)
+                       heads_dev, n_heads_nz, lh0, sm.lens, sm.S_max, rows, M, colpart, sm.B)
     if (n_heads_nz <= 2) CIH_APC(2, 8);
     else if (n_heads_nz <= 4) CIH_APC(4, 8);
     else if (n_heads_nz <= 7) CIH_APC(7, 4);
@@ -406,12 +407,10 @@ hipError_t launch_apc_layer(const float *P, int64_t pb, int64_t ph, int H, int l
     else if (n_heads_nz <= 20) CIH_APC(20, 2);
     else CIH_APC(APC_HMAX, 2);
 #undef CIH_APC
-    hipLaunchKernelGGL(k_apc_r, dim3((n_max + 63) / 64, n_heads_nz, sm.B), dim3(256), 0, st, rowsum, colpart, H, l,
-                       heads_dev, n_heads_nz, sm.lens, sm.S_max, rows, r, sm.B);
     return hipGetLastError();
 }
 
-// coef[t][b] = w_lh / T_lh of layer-head lh = lhs[t] (0 when |T| <= 1e-12), T = sum_i r_i
+// coef[k][b] = w_lh / T_lh of layer-head lh = lhs[k] (0 when |T| <= 1e-12), T = sum_i r_i
 __global__ __launch_bounds__(256) void k_apc_coef(const float *__restrict__ r, const float *__restrict__ w,
                                                   const int *__restrict__ lhs, const int *__restrict__ lens, int S_max,
                                                   int B, float *__restrict__ coef) {
@@ -419,7 +418,7 @@ __global__ __launch_bounds__(256) void k_apc_coef(const float *__restrict__ r, c
     const int n = lens[b] - 2, n_max = S_max - 2;
     __shared__ float red[4];
     float s = 0.0f;
-    for (int i = threadIdx.x; i < n; i += 256) s += r[((size_t)lh * B + b) * n_max + i];
+    for (int i = threadIdx.x; i < n; i += 256) s += r[((size_t)blockIdx.x * B + b) * n_max + i];
     s = wave_sum(s);
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
     __syncthreads();
@@ -436,8 +435,7 @@ __global__ __launch_bounds__(256) void k_apc_coef(const float *__restrict__ r, c
 // form: corr = fma(c, r_i * r_j, corr) in layer-head order, skipping c == 0.
 constexpr int APC_FT = 64, APC_FL = 64;
 __global__ __launch_bounds__(256) void k_apc_final(const float *__restrict__ M, const float *__restrict__ r,
-                                                   const float *__restrict__ coef, const int *__restrict__ lhs,
-                                                   int nlh, const int *__restrict__ lens, int S_max, int B,
+                                                   const float *__restrict__ coef, int nlh, const int *__restrict__ lens, int S_max, int B,
                                                    float bias, float *__restrict__ out, int n_stride) {
     const int b = blockIdx.z, i0 = blockIdx.y * APC_FT, j0 = blockIdx.x * APC_FT;
     const int n = lens[b] - 2, n_max = S_max - 2;
@@ -455,7 +453,7 @@ __global__ __launch_bounds__(256) void k_apc_final(const float *__restrict__ M, 
         for (int e = tid; e < APC_FL * APC_FT; e += 256) {
             const int t = lh0 + e / APC_FT, x = e % APC_FT;
             const bool in = t < nlh;
-            const float *rr = r + ((size_t)lhs[in ? t : 0] * B + b) * n_max;
+            const float *rr = r + ((size_t)(in ? t : 0) * B + b) * n_max;
             ri[e / APC_FT][x] = in && i0 + x < n ? rr[i0 + x] : 0.0f;
             rj[e / APC_FT][x] = in && j0 + x < n ? rr[j0 + x] : 0.0f;
         }
@@ -489,15 +487,19 @@ __global__ __launch_bounds__(256) void k_apc_final(const float *__restrict__ M, 
     }
 }
 
-hipError_t launch_apc_finalize(const float *M, const float *r, float *coef, const float *w_dev, const int *lhs_dev,
-                               int nlh, SeqMeta sm, float bias, float *contacts, int n_stride, hipStream_t st) {
+hipError_t launch_apc_finalize(const float *M, const float *rowsum, const float *colpart, float *r, float *coef,
+                               const float *w_dev, const int *lhs_dev, int nlh, int H, SeqMeta sm, float bias,
+                               float *contacts, int n_stride, hipStream_t st) {
     if (sm.S_max < 3) return hipSuccess;
     const int n_max = sm.S_max - 2;
-    if (nlh > 0)
+    if (nlh > 0) {
+        hipLaunchKernelGGL(k_apc_r, dim3((n_max + 63) / 64, nlh, sm.B), dim3(256), 0, st, rowsum, colpart, H, lhs_dev,
+                           sm.lens, sm.S_max, apc_rows(sm.B, n_max), r, sm.B);
         hipLaunchKernelGGL(k_apc_coef, dim3(nlh, sm.B), dim3(256), 0, st, r, w_dev, lhs_dev, sm.lens, sm.S_max, sm.B,
                            coef);
+    }
     const int nt = (n_max + APC_FT - 1) / APC_FT;
-    hipLaunchKernelGGL(k_apc_final, dim3(nt, nt, sm.B), dim3(256), 0, st, M, r, coef, lhs_dev, nlh, sm.lens, sm.S_max, sm.B, bias,
+    hipLaunchKernelGGL(k_apc_final, dim3(nt, nt, sm.B), dim3(256), 0, st, M, r, coef, nlh, sm.lens, sm.S_max, sm.B, bias,
                        contacts, n_stride);
     return hipGetLastError();
 }

@@ -51,7 +51,7 @@ struct Workspace {
     float *rope_c = nullptr, *rope_s = nullptr;
     float *P = nullptr;                            // [maxB][H][maxS][maxS] probabilities scratch
     float *M = nullptr, *r = nullptr, *coef = nullptr;  // contacts
-    float *rowsum = nullptr, *colpart = nullptr;        // contacts: map row sums, column partial sums
+    float *rowsum = nullptr, *colpart = nullptr;        // contacts: map row sums [L][B][H][S], column partial sums
     PartialBuf part;                                    // partial sums of k-split GEMMs / GEMVs
     float *attp = nullptr;                              // partial results of key-split attention
     size_t attp_floats = 0;
