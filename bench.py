@@ -50,9 +50,8 @@ DTYPE_NOTE = ("GEMM activations as two f16 limbs (hi = f16(x), lo = f16(x - hi):
 
 def qgemm_name(wname, T, d):
     """Which quantized GEMM the forward's projections take at T tokens: the
-    LDS-staged kernel from 64 tokens on while the f16 copy of the quants is
-    there (its plan picks 64 x 64 tiles below about five per CU, the large
-    tiles above), or, for a model loaded with CIH_GEMM_F16=0, when even the
+    few-rows kernel from 9 to 48 tokens (to 64 for some projections), the
+    LDS-staged kernel above while the f16 copy of the quants is there, or, for a model loaded with CIH_GEMM_F16=0, when even the
     narrowest projection (N = d) gives a full round of 128 x 128 tiles; else
     the register-staged one (split-K for small T)."""
     env = os.environ.get
@@ -62,7 +61,9 @@ def qgemm_name(wname, T, d):
     elif env("CIH_GEMM_LDS") == "force":
         lds = True
     elif copy and env("CIH_GEMM_PLAN") != "0":
-        lds = T >= 64
+        if 8 < T <= 48 and env("CIH_GEMM_ROWS") != "0" and env("CIH_SPLITK") != "0":
+            return f"k_gemm_rows<{wname}> f16 MFMA, 2 limbs, W from the quants (QKV, Wo, FC1, FC2)"
+        lds = T > 48
     else:
         lds = -(-T // 128) * -(-d // 128) >= 256
     if lds:
