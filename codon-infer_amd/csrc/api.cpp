@@ -291,10 +291,21 @@ int cih_model_reserve(cih_model *m, int32_t max_batch, int32_t max_seq_len, uint
                ok(dalloc(ws.kv_pos, T, dl)) && ok(dalloc(ws.kv_ti, B * ((S + 31) / 32) * 4, dl)) &&
                ok(hipMemset(ws.kv_img, 0, img));
     }
-    if (good && (flags & CIH_OUT_CONTACTS))
-        good = ok(dalloc(ws.M, B * n * n, dl)) && ok(dalloc(ws.r, L * H * B * n, dl)) &&
-               ok(dalloc(ws.coef, L * H * B, dl)) && ok(dalloc(ws.rowsum, L * B * H * S, dl)) &&
-               ok(dalloc(ws.colpart, apc_colpart_floats((int)B, std::max(m->n_lhs, 1), (int)n), dl));
+    if (good && (flags & CIH_OUT_CONTACTS)) {
+        // row and column sums of every weighted layer-head within 64 MiB each;
+        // beyond, of as many layers as that (one at least), which the forward
+        // then folds into r before it goes on (3B, B = 32, S = 1024: 71 MB of
+        // column sums for one layer at a time, 1.02 GB for all)
+        constexpr size_t budget = (size_t)16 << 20;
+        const size_t lhs = m->n_lhs, per = apc_colpart_floats((int)B, (int)n), rows = B * H * S;
+        size_t most = 1;
+        for (int nz : m->nz) most = std::max(most, (size_t)nz);
+        ws.apc_lhs = (int)std::max(most, std::min(lhs, budget / std::max(per, (size_t)1)));
+        ws.apc_layers = (int)std::max((size_t)1, std::min(L, budget / rows));
+        good = ok(dalloc(ws.M, B * n * n, dl)) && ok(dalloc(ws.r, lhs * B * n, dl)) &&
+               ok(dalloc(ws.coef, lhs * B, dl)) && ok(dalloc(ws.rowsum, ws.apc_layers * rows, dl)) &&
+               ok(dalloc(ws.colpart, ws.apc_lhs * per, dl));
+    }
     if (good && !(flags & CIH_IO_DEVICE)) {
         if (flags & CIH_OUT_LOGITS) good = good && ok(dalloc(ws.o_logits, T * V, dl));
         if (flags & CIH_OUT_HIDDEN) good = good && ok(dalloc(ws.o_hidden, T * d, dl));
@@ -482,10 +493,24 @@ int forward_impl(cih_model *m, const int32_t *tokens, const int32_t *lens, int32
         HIPCHK(launch_kv_setup(sm, (int)m->hd, H, ws.kv_tb, ws.kv_pk, ws.kv_pos, ws.kv_ti, ws.kv_img, st));
     }
 
-    for (int l = 0, lh = 0; l < L; l++) {
+    // contacts: the layer-heads of nonzero weight from g_lh and the layers from
+    // g_l on whose row and column sums wait in ws.rowsum and ws.colpart
+    int lh = 0, g_lh = 0, g_l = 0;
+    auto fold_apc = [&](int lh1) {
+        ProfScope ps(m, CIH_KC_OTHER, 0, 0);
+        return launch_apc_rows(ws.rowsum, ws.colpart, m->d_lhs + g_lh, lh1 - g_lh, g_l, H, sm,
+                               ws.r + (size_t)g_lh * B * n_max, st);
+    };
+    for (int l = 0; l < L; l++) {
         const Layer &ly = m->layers[l];
         const int lh0 = lh;  // this layer's first layer-head of nonzero contact weight
         lh += m->nz[l];
+        if (want_contacts && m->nz[l] > 0 && (lh - g_lh > ws.apc_lhs || l - g_l >= ws.apc_layers)) {
+            HIPCHK(fold_apc(lh0));
+            g_lh = lh0;
+            g_l = l;
+        }
+        float *rsum = want_contacts && m->nz[l] > 0 ? ws.rowsum + (size_t)(l - g_l) * B * H * S_max : nullptr;
         // probabilities: straight into the attention-map output when exported
         float *P = nullptr;
         int64_t pb = 0, ph = SS;
@@ -536,14 +561,13 @@ int forward_impl(cih_model *m, const int32_t *tokens, const int32_t *lens, int32
                 double fl = 0;
                 for (int b = 0; b < B; b++) fl += 4.0 * (double)lens[b] * lens[b] * d;
                 ProfScope ps(m, CIH_KC_ATTENTION, fl, 16.0 * T * d);
-                float *rsum = want_contacts && m->nz[l] > 0 ? ws.rowsum + (size_t)l * B * H * S_max : nullptr;
                 HIPCHK(launch_attention(ws.qkv, d, H, sm, ws.rope_c, ws.rope_s, ws.ao, af, P, pb, ph, rsum, ws.attp,
                                         ws.attp_floats, st, order, m->nz[l]));
             }
             if (want_contacts && m->nz[l] > 0) {
                 ProfScope ps(m, CIH_KC_OTHER, 0, 0);
                 HIPCHK(launch_apc_layer(P, pb, ph, H, l, m->d_contact_w, m->d_heads + (size_t)l * H, m->nz[l],
-                                        lh0, sm, ws.colpart, ws.M, st));
+                                        lh0 - g_lh, sm, ws.colpart, ws.M, st));
             }
             if (want_final && l == L - 1) {
                 ProfScope ps(m, CIH_KC_OTHER, 0, 0);
@@ -603,7 +627,6 @@ int forward_impl(cih_model *m, const int32_t *tokens, const int32_t *lens, int32
             double fl = 0;
             for (int b = 0; b < B; b++) fl += 4.0 * (double)lens[b] * lens[b] * d;
             ProfScope ps(m, CIH_KC_ATTENTION, fl, 16.0 * T * d);
-            float *rsum = want_contacts && m->nz[l] > 0 ? ws.rowsum + (size_t)l * B * H * S_max : nullptr;
             if (use_img)
                 HIPCHK(launch_attention_img(ws.qkv, d, H, sm, ws.kv_tb, ws.kv_img, ws.rope_c, ws.rope_s, ws.ao, af, P,
                                             pb, ph, rsum, ws.attp, ws.attp_floats, st, order, m->nz[l]));
@@ -614,7 +637,7 @@ int forward_impl(cih_model *m, const int32_t *tokens, const int32_t *lens, int32
         if (want_contacts && m->nz[l] > 0) {
             ProfScope ps(m, CIH_KC_OTHER, 0, 0);
             HIPCHK(launch_apc_layer(P, pb, ph, H, l, m->d_contact_w, m->d_heads + (size_t)l * H, m->nz[l],
-                                    lh0, sm, ws.colpart, ws.M, st));
+                                    lh0 - g_lh, sm, ws.colpart, ws.M, st));
         }
         if (want_final && l == L - 1) {
             ProfScope ps(m, CIH_KC_OTHER, 0, 0);
@@ -640,9 +663,10 @@ int forward_impl(cih_model *m, const int32_t *tokens, const int32_t *lens, int32
         if (want_layer) HIPCHK(launch_scatter_rows(ws.x, d, sm, t_layer + (size_t)l * S_max * d, (int64_t)L * S_max * d, st));
     }
     if (want_contacts) {
+        HIPCHK(fold_apc(lh));
         ProfScope ps(m, CIH_KC_OTHER, 0, 0);
-        HIPCHK(launch_apc_finalize(ws.M, ws.rowsum, ws.colpart, ws.r, ws.coef, m->d_contact_w, m->d_lhs, m->n_lhs, H,
-                                   sm, m->contact_b, t_contacts, n_max, st));
+        HIPCHK(launch_apc_finalize(ws.M, ws.r, ws.coef, m->d_contact_w, m->d_lhs, m->n_lhs, sm, m->contact_b,
+                                   t_contacts, n_max, st));
     }
     // final LayerNorm: state.x = LN_f(x) (lib.rs:5379-5387).  It also
     // reports a residual row that is no longer finite (the f16 limbs hold

@@ -443,20 +443,22 @@ hipError_t launch_head_mean(const float *P, int64_t pb, int64_t ph, int H, SeqMe
 
 // Contacts (APC).  For layer l, heads with w != 0, one read of the maps:
 //   M[b][i][j] += sum_h w_lh * P_lh[i+1][j+1]
-// and column partial sums of its heads, the layer-heads lh0 .. of nonzero
-// weight, in colpart (apc_colpart_floats(B, n_lhs, n_max) floats).
-size_t apc_colpart_floats(int B, int n_lhs, int n_max);
+// and column partial sums of its heads in colpart, layer-heads k0 .. of it
+// (apc_colpart_floats(B, n_max) floats each).
+size_t apc_colpart_floats(int B, int n_max);
 hipError_t launch_apc_layer(const float *P, int64_t pb, int64_t ph, int H, int l, const float *w_dev,
-                            const int *heads_dev, int n_heads_nz, int lh0, SeqMeta sm, float *colpart, float *M,
+                            const int *heads_dev, int n_heads_nz, int k0, SeqMeta sm, float *colpart, float *M,
                             hipStream_t st);
-// r[k][b][i] = rowsum[l][b][h][i+1] + sum_j P_lh[j+1][i+1] (residues only) for
-// layer-head lhs_dev[k] = l H + h, k < nlh (rowsum from launch_attention), then
+// r[k][b][i] = rowsum[l - l0][b][h][i+1] + sum_j P_lh[j+1][i+1] (residues only)
+// for layer-head lhs_dev[k] = l H + h, k < nlh: rowsum from launch_attention,
+// the column sums from colpart's layer-heads 0 .. nlh - 1.
+hipError_t launch_apc_rows(const float *rowsum, const float *colpart, const int *lhs_dev, int nlh, int l0, int H,
+                           SeqMeta sm, float *r, hipStream_t st);
 // contacts[b][i][j] = sigmoid(M_ij + M_ji - sum_lh (w_lh / T_lh) r_i r_j + bias)
 // over the nlh layer-heads of nonzero weight, lhs_dev their indices l H + h in
 // order.  coef: [nlh][B] scratch for w_lh / T_lh.
-hipError_t launch_apc_finalize(const float *M, const float *rowsum, const float *colpart, float *r, float *coef,
-                               const float *w_dev, const int *lhs_dev, int nlh, int H, SeqMeta sm, float bias,
-                               float *contacts, int n_stride, hipStream_t st);
+hipError_t launch_apc_finalize(const float *M, const float *r, float *coef, const float *w_dev, const int *lhs_dev,
+                               int nlh, SeqMeta sm, float bias, float *contacts, int n_stride, hipStream_t st);
 
 // DMS rows (pipeline.rs:152-172): for entry i, logits row meta[2i] of the
 // packed [T][V] logits and wild-type token meta[2i+1] give out[i][0..19] =

@@ -272,10 +272,11 @@ hipError_t launch_head_mean(const float *P, int64_t pb, int64_t ph, int H, SeqMe
 // Summed over heads: logit = M + M^T - sum_h (w_h / T_h) r_h r_h^T with
 // M = sum_h w_h A_h, and r_i = (row sum of A)_i + (column sum of A)_i.  The
 // attention kernel supplies the row sums; k_apc_tile reads each map once,
-// accumulating M and column partial sums of `rows` map rows; one k_apc_r after
-// the last layer adds those of every layer-head in order (a launch per layer
-// was 4.8 us each: 4% of a 650M L=257 forward).  M: [B][n_max][n_max], r:
-// [n_lhs][B][n_max] over the layer-heads of nonzero weight, n_max = S_max - 2.
+// accumulating M and column partial sums of `rows` map rows; one k_apc_r for
+// as many layers as the caller's buffers hold adds those of every layer-head
+// in order (a launch per layer was 4.8 us each: 4% of a 650M L=257 forward,
+// whose buffers hold all layers).  M: [B][n_max][n_max], r: [n_lhs][B][n_max]
+// over the layer-heads of nonzero weight, n_max = S_max - 2.
 constexpr int APC_HMAX = 40;     // most heads of any preset (3B)
 constexpr int APC_ROWS_MIN = 8;  // map rows per wave of k_apc_tile: 8, 16 or 32
 
@@ -290,11 +291,13 @@ static int apc_rows(int B, int n_max) {
     return rows;
 }
 
-// Enough for every call of at most B sequences and n_max residues: whole
-// 32-row tiles, or, where the rows were halved, fewer than 2 x 8 waves per CU
-// of 64 columns each.
-size_t apc_colpart_floats(int B, int n_lhs, int n_max) {
-    return (size_t)n_lhs * std::max((size_t)B * ((n_max + 31) / 32) * n_max, (size_t)2 * 8 * device_cus() * 64);
+// Enough for one layer-head in every call of at most B sequences and n_max
+// residues: whole 32-row tiles, or, where the rows were halved, fewer than
+// 2 x 8 waves per CU of 64 columns each, and no more than tiles of the fewest
+// rows take.
+size_t apc_colpart_floats(int B, int n_max) {
+    const auto tiles = [&](int rows) { return (size_t)B * ((n_max + rows - 1) / rows) * n_max; };
+    return std::max(tiles(32), std::min(tiles(APC_ROWS_MIN), (size_t)2 * 8 * device_cus() * 64));
 }
 
 // One wave = 64 residue columns x `rows` map rows.  HM >= nz heads per pass
@@ -306,7 +309,7 @@ size_t apc_colpart_floats(int B, int n_lhs, int n_max) {
 template <int HM, int R>
 __global__ __launch_bounds__(64) void k_apc_tile(const float *__restrict__ P, long long pb, long long ph, int H,
                                                  int l, const float *__restrict__ w, const int *__restrict__ heads,
-                                                 int nz, int lh0, const int *__restrict__ lens, int S_max, int rows,
+                                                 int nz, int k0, const int *__restrict__ lens, int S_max, int rows,
                                                  float *__restrict__ M, float *__restrict__ colpart, int B) {
     const int tile = blockIdx.x, b = blockIdx.z;
     const int n = lens[b] - 2, n_max = S_max - 2, ntiles = (n_max + rows - 1) / rows;
@@ -358,16 +361,17 @@ __global__ __launch_bounds__(64) void k_apc_tile(const float *__restrict__ P, lo
     }
 #pragma unroll
     for (int k = 0; k < HM; k++)
-        if (k < nz) colpart[(((size_t)(lh0 + k) * B + b) * ntiles + tile) * n_max + j] = cs[k];
+        if (k < nz) colpart[(((size_t)(k0 + k) * B + b) * ntiles + tile) * n_max + j] = cs[k];
 }
 
-// r[k][b][i] of layer-head lhs[k] = l H + h: rowsum[l][b][h][i+1] + column
+// r[k][b][i] of layer-head lhs[k] = l H + h: rowsum[l - l0][b][h][i+1] + column
 // partials of i in tile order, four waves of every fourth group of 8 tiles (8
 // loads in flight each) joined in wave order
 __global__ __launch_bounds__(256) void k_apc_r(const float *__restrict__ rowsum, const float *__restrict__ colpart,
-                                               int H, const int *__restrict__ lhs, const int *__restrict__ lens,
-                                               int S_max, int rows, float *__restrict__ r, int B) {
-    const int b = blockIdx.z, k = blockIdx.y, l = lhs[k] / H, h = lhs[k] % H;
+                                               int H, const int *__restrict__ lhs, int l0,
+                                               const int *__restrict__ lens, int S_max, int rows,
+                                               float *__restrict__ r, int B) {
+    const int b = blockIdx.z, k = blockIdx.y, l = lhs[k] / H - l0, h = lhs[k] % H;
     const int n = lens[b] - 2, n_max = S_max - 2, ntiles = (n_max + rows - 1) / rows;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, i = blockIdx.x * 64 + lane;
     __shared__ float part[3][64];
@@ -391,7 +395,7 @@ __global__ __launch_bounds__(256) void k_apc_r(const float *__restrict__ rowsum,
 }
 
 hipError_t launch_apc_layer(const float *P, int64_t pb, int64_t ph, int H, int l, const float *w_dev,
-                            const int *heads_dev, int n_heads_nz, int lh0, SeqMeta sm, float *colpart, float *M,
+                            const int *heads_dev, int n_heads_nz, int k0, SeqMeta sm, float *colpart, float *M,
                             hipStream_t st) {
     if (n_heads_nz <= 0 || sm.S_max < 3) return hipSuccess;
     if (n_heads_nz > APC_HMAX || H > APC_HMAX) return hipErrorInvalidValue;
@@ -399,7 +403,7 @@ hipError_t launch_apc_layer(const float *P, int64_t pb, int64_t ph, int H, int l
     const dim3 tg((n_max + rows - 1) / rows, (n_max + 63) / 64, sm.B);
 #define CIH_APC(HM, R)                                                                                              \
     hipLaunchKernelGGL((k_apc_tile<HM, R>), tg, dim3(64), 0, st, P, (long long)pb, (long long)ph, H, l, w_dev,       \
-                       heads_dev, n_heads_nz, lh0, sm.lens, sm.S_max, rows, M, colpart, sm.B)
+                       heads_dev, n_heads_nz, k0, sm.lens, sm.S_max, rows, M, colpart, sm.B)
     if (n_heads_nz <= 2) CIH_APC(2, 8);
     else if (n_heads_nz <= 4) CIH_APC(4, 8);
     else if (n_heads_nz <= 7) CIH_APC(7, 4);
@@ -487,17 +491,22 @@ __global__ __launch_bounds__(256) void k_apc_final(const float *__restrict__ M, 
     }
 }
 
-hipError_t launch_apc_finalize(const float *M, const float *rowsum, const float *colpart, float *r, float *coef,
-                               const float *w_dev, const int *lhs_dev, int nlh, int H, SeqMeta sm, float bias,
-                               float *contacts, int n_stride, hipStream_t st) {
+hipError_t launch_apc_rows(const float *rowsum, const float *colpart, const int *lhs_dev, int nlh, int l0, int H,
+                           SeqMeta sm, float *r, hipStream_t st) {
+    if (nlh <= 0 || sm.S_max < 3) return hipSuccess;
+    const int n_max = sm.S_max - 2;
+    hipLaunchKernelGGL(k_apc_r, dim3((n_max + 63) / 64, nlh, sm.B), dim3(256), 0, st, rowsum, colpart, H, lhs_dev, l0,
+                       sm.lens, sm.S_max, apc_rows(sm.B, n_max), r, sm.B);
+    return hipGetLastError();
+}
+
+hipError_t launch_apc_finalize(const float *M, const float *r, float *coef, const float *w_dev, const int *lhs_dev,
+                               int nlh, SeqMeta sm, float bias, float *contacts, int n_stride, hipStream_t st) {
     if (sm.S_max < 3) return hipSuccess;
     const int n_max = sm.S_max - 2;
-    if (nlh > 0) {
-        hipLaunchKernelGGL(k_apc_r, dim3((n_max + 63) / 64, nlh, sm.B), dim3(256), 0, st, rowsum, colpart, H, lhs_dev,
-                           sm.lens, sm.S_max, apc_rows(sm.B, n_max), r, sm.B);
+    if (nlh > 0)
         hipLaunchKernelGGL(k_apc_coef, dim3(nlh, sm.B), dim3(256), 0, st, r, w_dev, lhs_dev, sm.lens, sm.S_max, sm.B,
                            coef);
-    }
     const int nt = (n_max + APC_FT - 1) / APC_FT;
     hipLaunchKernelGGL(k_apc_final, dim3(nt, nt, sm.B), dim3(256), 0, st, M, r, coef, nlh, sm.lens, sm.S_max, sm.B, bias,
                        contacts, n_stride);

@@ -51,7 +51,8 @@ struct Workspace {
     float *rope_c = nullptr, *rope_s = nullptr;
     float *P = nullptr;                            // [maxB][H][maxS][maxS] probabilities scratch
     float *M = nullptr, *r = nullptr, *coef = nullptr;  // contacts
-    float *rowsum = nullptr, *colpart = nullptr;        // contacts: map row sums [L][B][H][S], column partial sums
+    float *rowsum = nullptr, *colpart = nullptr;  // contacts: map row sums [apc_layers][B][H][S], column partial sums
+    int apc_lhs = 0, apc_layers = 0;              // layer-heads that colpart and layers that rowsum hold
     PartialBuf part;                                    // partial sums of k-split GEMMs / GEMVs
     float *attp = nullptr;                              // partial results of key-split attention
     size_t attp_floats = 0;

@@ -138,6 +138,77 @@ def test_contacts_sparse_heads(H, hd, dtype, lens):
     assert np.abs(got[0]["logits"] - got[1]["logits"]).max() <= 1e-5 * max(1.0, np.abs(got[1]["logits"]).max())
 
 
+def free_bytes():
+    free, total = ctypes.c_size_t(), ctypes.c_size_t()
+    hip = ctypes.CDLL("libamdhip64.so")
+    assert hip.hipDeviceSynchronize() == 0
+    assert hip.hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+    return free.value
+
+
+def dense_head_model(L, H, hd, weights, **reserve):
+    cfg = ch.EsmConfig(H * hd, 64, L, H)
+    w = ch.EsmWeights.random(cfg, seed=L + H, std=0.05, bias_std=0.02)
+    return cfg, w, ch.GpuModel(cfg, w, contact_head=(weights, np.float32(-1.0)), **reserve)
+
+
+def test_contacts_workspace_follows_the_call():
+    """What contacts add to a workspace, all 288 layer-heads weighted: next to nothing for one peptide (six buffers of
+    less than a 2 MiB page each), and for 8 x 512 tokens, beyond the maps' own scratch, 64 MiB of row and of column sums
+    at most (map sums and r: 13 MB)."""
+    head = np.random.default_rng(0).normal(0, 3, (12, 24)).astype(np.float32)
+    cfg, w, m = dense_head_model(12, 24, 16, head)
+    for b, s, most in ((1, 10, 16 << 20), (8, 512, 8 * 24 * 512 * 512 * 4 + (160 << 20))):
+        got = []
+        for flags in (ch.OUT_LOGITS, ch.OUT_LOGITS | ch.OUT_CONTACTS):
+            m.reserve(b, s, flags | ch.IO_DEVICE)
+            got.append(free_bytes())
+        print(f"B={b} S={s}: contacts add {(got[0] - got[1]) >> 20} MiB", flush=True)
+        assert got[0] - got[1] <= most, (b, s)
+    m.close()
+
+
+@pytest.mark.parametrize("L,H,per_layer,lens", [
+    (5, 20, 20, [1024, 33, 20, 40]),   # 64 layer-heads of column sums: folded after three layers
+    (11, 40, 1, [700] + [5] * 63)])    # nine layers of row sums
+def test_contacts_folded_in_groups_of_layers(L, H, per_layer, lens):
+    """Batches whose row and column sums do not all fit the workspace, against the oracle."""
+    cfg = ch.EsmConfig(16 * H, 64, L, H)
+    w = ch.EsmWeights.random(cfg, seed=L, std=0.05, bias_std=0.02)
+    rng = np.random.default_rng(H)
+    head = np.zeros((L, H), np.float32)
+    for row in head:
+        row[rng.permutation(H)[:per_layer]] = rng.normal(0, 3, per_layer)
+    seqs = [rand_tokens(rng, n - 2) for n in lens]
+    check_batch(cfg, w, seqs, ch.OUT_LOGITS | ch.OUT_CONTACTS, contact=(head, np.float32(-1.0)))
+
+
+def test_contacts_in_a_larger_workspace():
+    """A workspace reserved for more sequences and residues than the call gives the bits of one reserved for it."""
+    head = np.random.default_rng(1).normal(0, 3, (3, 20)).astype(np.float32)
+    rng = np.random.default_rng(2)
+    seqs = [rand_tokens(rng, n - 2) for n in (300, 41, 3)]
+    flags = ch.OUT_LOGITS | ch.OUT_CONTACTS
+    got = []
+    for b, s in ((3, 300), (9, 777)):
+        cfg, w, m = dense_head_model(3, 20, 24, head, max_batch=b, max_len=s, outputs=flags)
+        got.append(m.forward(seqs, flags))
+        m.close()
+    for i, t in enumerate(seqs):
+        n = len(t) - 2
+        assert np.array_equal(got[0]["contacts"][i, :n, :n], got[1]["contacts"][i, :n, :n]), i
+
+
+@pytest.mark.parametrize("n", [3, 40, 300])
+def test_contacts_of_an_all_zero_head(n):
+    """No weighted layer-head: every contact is sigmoid(bias)."""
+    cfg, w, m = dense_head_model(2, 4, 32, np.zeros((2, 4), np.float32), max_len=n,
+                                 outputs=ch.OUT_LOGITS | ch.OUT_CONTACTS)
+    got = m.forward([rand_tokens(np.random.default_rng(n), n - 2)], ch.OUT_LOGITS | ch.OUT_CONTACTS)["contacts"]
+    m.close()
+    assert np.abs(got[0, :n - 2, :n - 2] - 1.0 / (1.0 + np.exp(1.0))).max() <= 1e-6
+
+
 def test_contacts_forty_heads():
     """Contacts with more than 20 weighted heads per layer (the 3B and 15B
     head count, 40): the map reader's 40-head pass, with a few zero-weight
