@@ -1375,7 +1375,12 @@ bool gemm_lds_plan(const DevMatrix &W, int a_fmt, int M, int epi, size_t part_fl
     const long cus = device_cus();
     const long t64 = (long)((M + 63) / 64) * ((W.N + 63) / 64), t128 = (long)((M + 127) / 128) * ((W.N + 127) / 128);
     const int KB = W.K / 32;
-    const bool can_split = epi == EPI_RESIDUAL && part_floats > 0 && !(ke && !strcmp(ke, "0"));
+    // k-splits whose partial sums part_floats holds: a rule that wants more does
+    // not apply (its tile, unsplit, would leave most of the CUs idle: 3B FC2 at
+    // 820 rows 56 workgroups of 320 blocks), but for the 64 x 64 tiles, which
+    // take as many as there is room for
+    const bool split_on = epi == EPI_RESIDUAL && !(ke && !strcmp(ke, "0"));
+    const int smax = split_on ? (int)std::min<size_t>(part_floats / ((size_t)M * W.N), 6) : 0;
     int tile, S = 1;
     // 128 x 320 tiles in 2 to 4 k-splits that fill 80% of the CUs or more, with
     // 40 blocks or more each (fewer: the fold costs what they gain).  GEMM and
@@ -1385,24 +1390,22 @@ bool gemm_lds_plan(const DevMatrix &W, int a_fmt, int M, int epi, size_t part_fl
     // 136, 2600 rows 83 / 92, 1616 rows 62 / 68; 3B Wo at 2048 rows 77 / 81.
     // Below 80%: 3B FC2 at 1500 rows (192 workgroups) 194 / 178.
     const long t320 = (long)((M + 127) / 128) * ((W.N + 319) / 320);
-    int s320 = can_split && !W.kx ? (int)std::min<long>(cus / t320, 4) : 1;
-    if (s320 >= 2 && (t320 * s320 * 10 < cus * 8 || KB / s320 < 40)) s320 = 1;
+    int s320 = !W.kx ? (int)std::min<long>(cus / t320, 4) : 1;
+    if (s320 > smax || t320 * s320 * 10 < cus * 8 || KB / s320 < 40) s320 = 1;
+    // deep projections: 64 x 128 tiles for at most 100 tiles of 128 x 128
+    const bool deep = KB >= 160 && t128 * 256 > 25 * cus && t128 < cus;
+    const int sdeep = t128 * 256 <= 100 * cus ? 3 : (int)std::min<long>(2 * cus / t128, 3);
     if (const int forced = tile_env(epi)) {
         tile = forced;
     } else if (s320 >= 2) {
         tile = LDS_TILE_128x320;
         S = s320;
-    } else if (can_split && KB >= 160 && t128 * 256 > 25 * cus && t128 < cus) {
-        if (t128 * 256 <= 100 * cus) {
-            tile = LDS_TILE_64x128;
-            S = 3;
-        } else {
-            tile = LDS_TILE_128x128;
-            S = (int)std::min<long>(2 * cus / t128, 3);
-        }
-    } else if (can_split && 2 * t64 <= cus) {
+    } else if (deep && sdeep <= smax) {
+        tile = t128 * 256 <= 100 * cus ? LDS_TILE_64x128 : LDS_TILE_128x128;
+        S = sdeep;
+    } else if (smax >= 2 && 2 * t64 <= cus) {
         tile = LDS_TILE_64x64;
-        S = (int)std::max<long>(1, std::min<long>({cus / t64, 6, KB / 4}));
+        S = (int)std::max<long>(1, std::min<long>({cus / t64, smax, KB / 4}));
         if (S == 5) S = 4;
     } else {
         tile = tile_time(M, W.N, KB, W.kx != 0, epi);
@@ -1410,7 +1413,6 @@ bool gemm_lds_plan(const DevMatrix &W, int a_fmt, int M, int epi, size_t part_fl
     // a pair copy (W.kx): the 64-row tiles and 128 x 320 (the others keep the
     // register-staged pair path)
     if (W.kx && tile != LDS_TILE_64x64 && tile != LDS_TILE_64x128 && tile != LDS_TILE_128x320) return false;
-    while (S > 1 && (size_t)S * M * W.N > part_floats) S--;
     if (S > 1) {
         p.kps = (KB + S - 1) / S;
         S = (KB + p.kps - 1) / p.kps;
