@@ -1353,7 +1353,7 @@ hipError_t launch_gemm_lds_split(const DevMatrix &W, const void *X, int M, const
 //   * those with K >= 5120 (160 blocks) from 25 tiles of 128 x 128 on (fewer:
 //     the 64 x 64 rule below): up to 100 such tiles, 64 x 128 tiles in 3
 //     k-splits; fewer 128 x 128 tiles than CUs, those in min(2 CUs / tiles,
-//     3) splits;
+//     3) splits (neither where one round of unsplit tiles does, one_round);
 //   * those with at most half as many 64 x 64 tiles as CUs: that tile in
 //     min(CUs / tiles, 6, blocks / 4) splits (5 -> 4);
 //   * else the tile whose fullest CU is done first (tile_time); 64 x 64 tiles
@@ -1382,6 +1382,15 @@ bool gemm_lds_plan(const DevMatrix &W, int a_fmt, int M, int epi, size_t part_fl
     const bool split_on = epi == EPI_RESIDUAL && !(ke && !strcmp(ke, "0"));
     const int smax = split_on ? (int)std::min<size_t>(part_floats / ((size_t)M * W.N), 6) : 0;
     int tile, S = 1;
+    // Deep projections whose 64 x 128 tiles fit one round of the CUs unsplit and
+    // take three in three k-splits: unsplit (GEMM and the LayerNorm after it,
+    // us, against the split rules below: 650M FC2 at 1100 rows 54 / 57, 1281
+    // rows 54 / 64, 1536 rows 57 / 65, 1600 rows 58 / 60; 3B FC2 at 560 rows 98
+    // / 100, 700 rows 102 / 114; pair copies of 650M FC2 at 1300 rows 99 / 139,
+    // of 150M FC2 at 2300 rows 54 / 56).  Two rounds: 650M FC2 at 1000 rows 52 /
+    // 48, 3B FC2 at 500 rows 98 / 80.
+    const long t64n = (long)((M + 63) / 64) * ((W.N + 127) / 128);
+    const bool one_round = KB >= 160 && t64n <= cus && 3 * t64n > 2 * cus;
     // 128 x 320 tiles in 2 to 4 k-splits that fill 80% of the CUs or more, with
     // 40 blocks or more each (fewer: the fold costs what they gain).  GEMM and
     // the LayerNorm that adds the splits, us, against the best of the other
@@ -1391,9 +1400,9 @@ bool gemm_lds_plan(const DevMatrix &W, int a_fmt, int M, int epi, size_t part_fl
     // Below 80%: 3B FC2 at 1500 rows (192 workgroups) 194 / 178.
     const long t320 = (long)((M + 127) / 128) * ((W.N + 319) / 320);
     int s320 = !W.kx ? (int)std::min<long>(cus / t320, 4) : 1;
-    if (s320 > smax || t320 * s320 * 10 < cus * 8 || KB / s320 < 40) s320 = 1;
+    if (s320 > smax || one_round || t320 * s320 * 10 < cus * 8 || KB / s320 < 40) s320 = 1;
     // deep projections: 64 x 128 tiles for at most 100 tiles of 128 x 128
-    const bool deep = KB >= 160 && t128 * 256 > 25 * cus && t128 < cus;
+    const bool deep = KB >= 160 && t128 * 256 > 25 * cus && t128 < cus && !one_round;
     const int sdeep = t128 * 256 <= 100 * cus ? 3 : (int)std::min<long>(2 * cus / t128, 3);
     if (const int forced = tile_env(epi)) {
         tile = forced;

@@ -272,7 +272,8 @@ def test_lm_head_limb_handoff_is_bit_identical(case, monkeypatch):
     (1280, 5120, 20, [517, 513, 510]),     # FC2 in 4 splits of 40 blocks
     (1280, 5120, 20, [520] * 5),           # FC2 in 3 splits, the last shorter
     (480, 1920, 20, [512, 131, 387, 254, 449, 173, 318, 505]),  # FC1 on 64 x 128 tiles past 1280 tiles of 64 x 64
-    (640, 2560, 20, [700, 700, 701])])
+    (640, 2560, 20, [700, 700, 701]),
+    (640, 5120, 20, [641, 700, 780])])    # FC2 unsplit in one round of 64 x 128 tiles
 @pytest.mark.parametrize("dtype", [1, 2])
 def test_plan_matches_the_routes_without_it(d, F, H, lens, dtype, monkeypatch):
     """Tiles and splits of the plan against the routes without it (CIH_GEMM_PLAN=0): the same products summed in
