@@ -406,7 +406,7 @@ int cih_decoder_create(cih_model *m, int32_t n_slots, int32_t max_len, int32_t m
                 dalloc(dc->d_tokens, R, al) == hipSuccess && dalloc(dc->d_rows, 2 * R, al) == hipSuccess &&
                 dalloc(dc->d_cu, R, al) == hipSuccess && dalloc(dc->d_lens, R, al) == hipSuccess &&
                 dalloc(dc->d_flag, 1, al) == hipSuccess;
-    dc->part.floats = model_part_floats(m);
+    dc->part.floats = model_part_floats(m, R);  // a prompt's residual projections split over K too
     good = good && dalloc(dc->part.part, dc->part.floats, al) == hipSuccess &&
            hipHostMalloc((void **)&dc->h_meta, (3 * R + 1) * sizeof(int)) == hipSuccess &&
            hipHostMalloc((void **)&dc->h_logits, R * V * sizeof(float)) == hipSuccess;

@@ -12,6 +12,7 @@ import pytest
 
 import codon_hip as ch
 import cpu_ref as cr
+from test_gpu_forward import free_bytes
 
 pytestmark = pytest.mark.gpu
 TOL = 1e-3
@@ -320,5 +321,33 @@ def test_decode_attention_past_one_sweep(hd, rows):
     for p in sorted({1, 2, step - 1, step, step + 1, rows - 1} | ({2 * step, 2 * step + 1} if 2 * step + 1 < rows else set())):
         one = dec.decode([0], [toks[p]], [p])[0]
         assert np.abs(one - ref[p]).max() <= 1e-3, p
+    dec.close()
+    m.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("d,F,rows", [(2560, 2560, 2048), (1280, 5120, 4096)])
+def test_prefill_has_room_for_its_splits(d, F, rows, monkeypatch):
+    """A decoder's partial buffer holds four k-splits of 256 tiles of 128 x 128 (67 MB, what the split residual
+    projections of a long prompt leave to the LayerNorm): the memory it takes beyond caches and activations (three
+    quarters of that, as the count is of whole pages and of what the runtime had at hand), and the prompt's logits
+    against those of the routes without the plan (1e-5 of the largest: FP32 sums in another order)."""
+    cfg = ch.EsmConfig(d, F, 1, d // 64, max_seq_len=rows)
+    w = ch.EsmWeights.random(cfg, seed=rows, std=0.02, bias_std=0.02).quantize_q4()
+    m = ch.GpuModel(cfg, w, max_batch=1, max_len=16)
+    free = [free_bytes()]
+    dec = ch.GpuDecoder(m, n_slots=1, max_len=rows, max_rows=rows)
+    free.append(free_bytes())
+    activations = 4 * rows * (2 * d + 3 * d + 3 * d + F)  # caches; x, xb, ao; qkv; h
+    assert rows * d >= 256 * 128 * 128
+    assert free[0] - free[1] >= activations + 3 * 4 * 256 * 128 * 128
+    toks = np.concatenate([[0], 4 + np.random.default_rng(rows).integers(0, 20, rows - 1)]).astype(np.int32)
+    got = []
+    for env in (None, "0"):
+        if env:
+            monkeypatch.setenv("CIH_GEMM_PLAN", env)
+        got.append(dec.decode(np.zeros(rows), toks, np.arange(rows)))
+    assert np.isfinite(got[0]).all()
+    assert np.abs(got[0] - got[1]).max() <= 1e-5 * max(1.0, np.abs(got[1]).max())
     dec.close()
     m.close()
