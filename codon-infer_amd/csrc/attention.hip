@@ -444,11 +444,15 @@ __device__ __forceinline__ void split8_mix(const float *v, f16x8 &hi, f16x8 &lo)
 
 // Work items: (sequence, head, query block) tasks, task = (b * H + h) * nq + qb,
 // one workgroup each for the first nfull; every later task is split into
-// nsplit ranges of whole 32-key tiles (one workgroup each, ONEPASS only)
+// nsplit ranges of whole 32-key tiles (one workgroup each, ATT_ONEPASS only)
 // that leave their unnormalized output, running max and sum in part for
-// k_attention_merge.
-template <int HD, bool ONEPASS, int NTH = 256>
-__global__ __launch_bounds__(NTH, ONEPASS || HD <= 32 ? 4 : 2) void k_attention_h(const float *__restrict__ qkv, int d, const int *__restrict__ cu,
+// k_attention_merge.  ATT_MIXED: head slots below nexp (of order) take the two
+// passes and export, the others one pass, with the bits of the kernels of one
+// kind (its small workgroups run one wave per SIMD and need no more registers
+// spared for others).
+template <int HD, int MODE, int NTH = 256>
+__global__ __launch_bounds__(NTH, MODE == ATT_ONEPASS || (HD <= 32 && (MODE == ATT_EXPORT || NTH > 128)) ? 4 : 2)
+void k_attention_h(const float *__restrict__ qkv, int d, const int *__restrict__ cu,
                                                      const int *__restrict__ lens, int S_max,
                                                      const float *__restrict__ rc, const float *__restrict__ rsn,
                                                      void *__restrict__ out, int out_fmt, float *__restrict__ P,
@@ -465,7 +469,7 @@ __global__ __launch_bounds__(NTH, ONEPASS || HD <= 32 ? 4 : 2) void k_attention_
     constexpr int DT = VW / 32;
     constexpr int K_LD = HDP + 8;             // f16 per LDS key row (16-byte aligned, padded)
     constexpr int V_LD = 32 + 8;              // f16 per LDS dim row of the transposed V tile
-    constexpr int NBUF = ONEPASS ? 1 : 2;     // the export kernel double-buffers its tiles
+    constexpr int NBUF = MODE == ATT_ONEPASS ? 1 : 2;  // the two-pass form double-buffers its tiles
     constexpr int KBUF = 32 * K_LD, VBUF = VW * V_LD;
     __shared__ __attribute__((aligned(16))) _Float16 Kh[NBUF * KBUF], Kl[NBUF * KBUF];
     __shared__ __attribute__((aligned(16))) _Float16 Vh[NBUF * VBUF], Vl[NBUF * VBUF];
@@ -478,9 +482,8 @@ __global__ __launch_bounds__(NTH, ONEPASS || HD <= 32 ? 4 : 2) void k_attention_
         ks = t % nsplit;
         ns = nsplit;
     }
-    // head slot: the order of heads, exported ones first (null: all in order)
     const int qb = task % nq, slot = (task / nq) % H, b = task / nq / H;
-    const int h = order ? order[slot] : slot;
+    const int h = MODE == ATT_MIXED ? order[slot] : slot;
     const int len = lens[b], base = cu[b];
     const int qblk = qb * (NTH / 2);  // 32 queries per wave
     if (qblk >= len) return;
@@ -613,7 +616,7 @@ __global__ __launch_bounds__(NTH, ONEPASS || HD <= 32 ? 4 : 2) void k_attention_
 #pragma unroll
         for (int q = 0; q < 16; q++) oacc[t][q] = 0.0f;
     float out_scale;
-    if constexpr (ONEPASS) {
+    if constexpr (MODE == ATT_ONEPASS) {
         // One pass, online softmax (see k_attention) in base 2: the query is
         // pre-scaled by log2(e) / sqrt(hd) so every exponential is one
         // v_exp_f32, and the MFMAs start from -m, so their results are the
@@ -656,7 +659,8 @@ __global__ __launch_bounds__(NTH, ONEPASS || HD <= 32 ? 4 : 2) void k_attention_
     } else {
         // Two passes over the keys (the exported probabilities are final, so
         // the row max and sum come first), base-2 exponentials of the
-        // pre-scaled scores.  With one 32-query wave per SIMD slot and few
+        // pre-scaled scores, or, for a head without an export, the one pass
+        // above.  With one 32-query wave per SIMD slot and few
         // waves, a tile's global loads are the critical path: they go to
         // registers one tile ahead (fetch) and into LDS as f16 limbs after the
         // barrier (stage), so tile t+1 is in flight while tile t is computed.
@@ -746,50 +750,63 @@ __global__ __launch_bounds__(NTH, ONEPASS || HD <= 32 ? 4 : 2) void k_attention_
                 body(kt0);
             }
         };
-        // pass 1: running max / sum of exp per lane
-        float m = -INFINITY, l = 0.0f;
-        sweep(false, [&](int kt0) __attribute__((always_inline)) {
-            f32x16 acc;
-            scores(acc, 0.0f);
-            float sv[16];
-            float tmax = -INFINITY;
+        if (MODE == ATT_MIXED && slot >= nexp) {
+            float m = -INFINITY, l = 0.0f;
+            sweep(true, [&](int kt0) __attribute__((always_inline)) {
+                online_tile<DT, true>(m, l, oacc, kt0, len, hh, [&](f32x16 &acc, float c0) { scores(acc, c0); },
+                                      [&](const float (&p)[16]) { pv(oacc, p); });
+            });
+            out_scale = 1.0f / (l + __shfl_xor(l, 32));
+        } else {
+            // vmcnt(0): nothing is in flight here, but the compiler, which shares
+            // registers with the branch above, would wait for all loads inside
+            // pass 1's loop instead (its tile fetched ahead too: 35M B = 3 (512,
+            // 300, 257) 38.4 -> 43.0 us per layer)
+            if constexpr (MODE == ATT_MIXED) __builtin_amdgcn_s_waitcnt(0x0f70);
+            // pass 1: running max / sum of exp per lane
+            float m = -INFINITY, l = 0.0f;
+            sweep(false, [&](int kt0) __attribute__((always_inline)) {
+                f32x16 acc;
+                scores(acc, 0.0f);
+                float sv[16];
+                float tmax = -INFINITY;
 #pragma unroll
-            for (int q = 0; q < 16; q++) {
-                const int key = kt0 + 8 * (q >> 2) + 4 * hh + (q & 3);
-                sv[q] = key < len ? acc[q] : -INFINITY;
-                tmax = fmaxf(tmax, sv[q]);
-            }
-            const float mn = fmaxf(m, tmax);
-            if (mn != -INFINITY) {
-                float sum = 0.0f;
+                for (int q = 0; q < 16; q++) {
+                    const int key = kt0 + 8 * (q >> 2) + 4 * hh + (q & 3);
+                    sv[q] = key < len ? acc[q] : -INFINITY;
+                    tmax = fmaxf(tmax, sv[q]);
+                }
+                const float mn = fmaxf(m, tmax);
+                if (mn != -INFINITY) {
+                    float sum = 0.0f;
 #pragma unroll
-                for (int q = 0; q < 16; q++) sum += __builtin_amdgcn_exp2f(sv[q] - mn);
-                l = l * __builtin_amdgcn_exp2f(m - mn) + sum;
-                m = mn;
-            }
-        });
-        const float mo = __shfl_xor(m, 32), lo = __shfl_xor(l, 32);
-        const float mx = fmaxf(m, mo);
-        const float inv_sum = 1.0f / (l * __builtin_amdgcn_exp2f(m - mx) + lo * __builtin_amdgcn_exp2f(mo - mx));
-        // pass 2: normalized probabilities, optional export, P.V
-        const bool exported = slot < nexp;
-        float *Prow = (P && exported && qi < len) ? P + b * pb + h * ph + (size_t)qi * S_max : nullptr;
-        float rs = 0.0f;  // sum of this query's probabilities over residue keys (contacts)
-        sweep(true, [&](int kt0) __attribute__((always_inline)) {
-            f32x16 acc;
-            scores(acc, 0.0f);
-            float p[16];
+                    for (int q = 0; q < 16; q++) sum += __builtin_amdgcn_exp2f(sv[q] - mn);
+                    l = l * __builtin_amdgcn_exp2f(m - mn) + sum;
+                    m = mn;
+                }
+            });
+            const float mo = __shfl_xor(m, 32), lo = __shfl_xor(l, 32);
+            const float mx = fmaxf(m, mo);
+            const float inv_sum = 1.0f / (l * __builtin_amdgcn_exp2f(m - mx) + lo * __builtin_amdgcn_exp2f(mo - mx));
+            // pass 2: normalized probabilities, optional export, P.V
+            float *Prow = (P && qi < len) ? P + b * pb + h * ph + (size_t)qi * S_max : nullptr;
+            float rs = 0.0f;  // sum of this query's probabilities over residue keys (contacts)
+            sweep(true, [&](int kt0) __attribute__((always_inline)) {
+                f32x16 acc;
+                scores(acc, 0.0f);
+                float p[16];
 #pragma unroll
-            for (int q = 0; q < 16; q++) {
-                const int key = kt0 + 8 * (q >> 2) + 4 * hh + (q & 3);
-                p[q] = key < len ? __builtin_amdgcn_exp2f(acc[q] - mx) * inv_sum : 0.0f;
-            }
-            if (Prow) store_p(Prow, p, kt0 + 4 * hh, len);
-            if (rowsum && exported) rs += tile_residue_sum(p, kt0, hh, len);
-            pv(oacc, p);
-        });
-        write_rowsum(exported ? rowsum : nullptr, rs, b, h, H, S_max, qi, len, hh);
-        out_scale = 1.0f;
+                for (int q = 0; q < 16; q++) {
+                    const int key = kt0 + 8 * (q >> 2) + 4 * hh + (q & 3);
+                    p[q] = key < len ? __builtin_amdgcn_exp2f(acc[q] - mx) * inv_sum : 0.0f;
+                }
+                if (Prow) store_p(Prow, p, kt0 + 4 * hh, len);
+                if (rowsum) rs += tile_residue_sum(p, kt0, hh, len);
+                pv(oacc, p);
+            });
+            write_rowsum(rowsum, rs, b, h, H, S_max, qi, len, hh);
+            out_scale = 1.0f;
+        }
     }
     if (qi < len) {
 #pragma unroll
@@ -1683,10 +1700,17 @@ hipError_t launch_attention(const float *qkv, int d, int H, SeqMeta sm, const fl
     hipLaunchKernelGGL((KER<HDV, ONE>), dim3((sm.S_max + 127) / 128, H, sm.B), dim3(256), 0, st, qkv, d, sm.cu, \
                        sm.lens, sm.S_max, rope_cos, rope_sin, out, out_fmt, P, (long long)pb, (long long)ph,     \
                        inv_scale, rowsum)
-#define CIH_ATT_H(HDV, ONE, NTH)                                                                                 \
-    hipLaunchKernelGGL((k_attention_h<HDV, ONE, NTH>), dim3(grid), dim3(NTH), 0, st, qkv, d, sm.cu, sm.lens,     \
+#define CIH_ATT_H(HDV, MODE, NTH)                                                                                \
+    hipLaunchKernelGGL((k_attention_h<HDV, MODE, NTH>), dim3(grid), dim3(NTH), 0, st, qkv, d, sm.cu, sm.lens,     \
                        sm.S_max, rope_cos, rope_sin, out, out_fmt, P, (long long)pb, (long long)ph, inv_scale, rowsum, \
                        H, nq, nfull, nsplit, part, order, nexp)
+#define CIH_ATT_HQ(HDV, MODE)                                                                                   \
+    do {                                                                                                        \
+        if (wide) CIH_ATT_H(HDV, MODE, 512);                                                                    \
+        else if (QB == 32) CIH_ATT_H(HDV, MODE, 64);                                                            \
+        else if (QB == 64) CIH_ATT_H(HDV, MODE, 128);                                                           \
+        else CIH_ATT_H(HDV, MODE, 256);                                                                         \
+    } while (0)
 #define CIH_ATT_XSK(HDV, KS, MODE)                                                                              \
     hipLaunchKernelGGL((k_attention_xs<HDV, KS, MODE>), dim3(t32), dim3(64 * KS), 0, st, qkv, d, sm.cu, sm.lens, \
                        sm.S_max, rope_cos, rope_sin, out, out_fmt, P, (long long)pb, (long long)ph, inv_scale,   \
@@ -1703,12 +1727,10 @@ hipError_t launch_attention(const float *qkv, int d, int H, SeqMeta sm, const fl
     else if (xsplit) CIH_ATT_XS(HDV, ATT_ONEPASS);                                                              \
     else if (fp32 && P) CIH_ATT_K(k_attention, HDV, false);                                                     \
     else if (fp32) CIH_ATT_K(k_attention, HDV, true);                                                           \
-    else if (P && wide) CIH_ATT_H(HDV, false, 512);                                                             \
-    else if (P && QB == 32) CIH_ATT_H(HDV, false, 64);                                                          \
-    else if (P && QB == 64) CIH_ATT_H(HDV, false, 128);                                                         \
-    else if (P) CIH_ATT_H(HDV, false, 256);                                                                     \
-    else if (wide) CIH_ATT_H(HDV, true, 512);                                                                   \
-    else CIH_ATT_H(HDV, true, 256);                                                                             \
+    else if (mixed) CIH_ATT_HQ(HDV, ATT_MIXED);                                                                 \
+    else if (P) CIH_ATT_HQ(HDV, ATT_EXPORT);                                                                    \
+    else if (wide) CIH_ATT_H(HDV, ATT_ONEPASS, 512);                                                            \
+    else CIH_ATT_H(HDV, ATT_ONEPASS, 256);                                                                      \
     if (nsplit > 1 && !xsplit) {                                                                                \
         const long n = (long)(tasks - nfull) * QB * (HDV / 4);                                                  \
         hipLaunchKernelGGL((k_attention_merge<HDV>), dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, part, \
@@ -1723,6 +1745,7 @@ hipError_t launch_attention(const float *qkv, int d, int H, SeqMeta sm, const fl
     }
 #undef CIH_ATT
 #undef CIH_ATT_H
+#undef CIH_ATT_HQ
 #undef CIH_ATT_XS
 #undef CIH_ATT_XSK
 #undef CIH_ATT_K

@@ -30,12 +30,13 @@ pytestmark = pytest.mark.gpu
 FLAGS = ch.OUT_LOGITS | ch.OUT_HIDDEN
 
 
-def run_paths(monkeypatch, cfg, w, seqs, flags):
+def run_paths(monkeypatch, cfg, w, seqs, flags, contact=None):
     """Outputs of the default path, the staged path (CIH_ATT_IMG=0), the prep
     kernel's images (CIH_ATT_IMG=prep) and the default path again."""
     monkeypatch.setenv("CIH_FORWARD_GRAPH", "0")
     monkeypatch.setenv("CIH_ATT_SPLIT", "0")
-    m = ch.GpuModel(cfg, w, max_batch=len(seqs), max_len=max(len(s) for s in seqs), outputs=flags)
+    m = ch.GpuModel(cfg, w, contact_head=contact, max_batch=len(seqs), max_len=max(len(s) for s in seqs),
+                    outputs=flags)
     out = {"default": m.forward(seqs, flags)}
     for tag, v in (("staged", "0"), ("prep", "prep")):
         monkeypatch.setenv("CIH_ATT_IMG", v)
@@ -94,6 +95,30 @@ def test_image_maps_vs_staged(monkeypatch, hd):
     e = float(np.abs(img["attn"][0, :, :, :S, :S] - ref["attn"]).max())
     print(f"hd {hd} maps vs oracle: {e:.2e}", flush=True)
     assert e <= 1e-5
+
+
+@pytest.mark.parametrize("n_seq", [1, 3, 6, 13])
+@pytest.mark.parametrize("hd", [64, 32, 24, 16])
+def test_image_contacts_vs_staged(monkeypatch, hd, n_seq):
+    """A sparse contact head, whose other heads take the one-pass softmax in both kernels, in the staged kernel's
+    32-, 64-, 128- and 256-query workgroups (1, 3, 6 and 13 sequences): contacts, logits and hidden states
+    bit-identical to the images', contacts of one sequence against the oracle."""
+    cfg = ch.EsmConfig(20 * hd, 20 * hd, 3, 20)
+    rng = np.random.default_rng(31 * hd + n_seq)
+    w = ch.EsmWeights.random(cfg, seed=hd, bias_std=0.02).quantize_q8()
+    head = np.zeros((3, 20), np.float32)
+    for row, n in zip(head, (3, 1, 12)):
+        row[rng.permutation(20)[:n]] = rng.normal(0, 3, n)
+    seqs = [rand_tokens(rng, int(rng.integers(200, 300))) for _ in range(n_seq)]
+    contact = (head, np.float32(-1.0))
+    out = run_paths(monkeypatch, cfg, w, seqs, FLAGS | ch.OUT_CONTACTS, contact)
+    for name in ("contacts", "logits", "hidden"):
+        for tag in ("staged", "default", "again"):
+            e = float(np.abs(out["prep"][name] - out[tag][name]).max())
+            assert np.array_equal(out["prep"][name], out[tag][name]), (name, tag, e)
+    n = len(seqs[0]) - 2
+    ref = cr.forward(cfg, w, seqs[0], 16, contacts=contact)
+    assert np.abs(out["prep"]["contacts"][0, :n, :n] - ref["contacts"]).max() <= 1e-4
 
 
 def test_graph_replay_with_another_tile_count(monkeypatch):
