@@ -241,8 +241,9 @@ def test_decode_attention_with_wo(hd, fmt, streams, monkeypatch):
 def overflow_model(where, seed):
     """A model whose reference results do not depend on one activation column
     that the f16 limbs cannot hold (~7e4, past f16's 65504): layer 0's LN1
-    column 37 (Q, K, V weights of that column zero) or the LM head's
-    LayerNorm column 37 (decoder weights of that column zero)."""
+    column 37 (Q, K, V weights of that column zero), its attention output
+    (Wo's zero) or FC1 output (FC2's zero), or the LM head's LayerNorm column
+    37 (decoder weights of that column zero)."""
     cfg = ch.EsmConfig(128, 512, 2, 4)
     w = ch.EsmWeights.random(cfg, seed=seed, bias_std=0.02)
     d, V, c = cfg.dim, cfg.vocab_size, 37
@@ -254,6 +255,14 @@ def overflow_model(where, seed):
             a = np.array(getattr(w, name), np.float32).reshape(cfg.n_layers, d, d)
             a[0, :, c] = 0.0
             setattr(w, name, a.ravel())
+    elif where in ("fc1", "attention"):
+        bias, weight, n = ("fc1_bias", "fc2_weight", cfg.hidden_dim) if where == "fc1" else ("bv", "wo", d)
+        b = np.array(getattr(w, bias), np.float32)
+        b[c] = 7.0e4
+        setattr(w, bias, b)
+        a = np.array(getattr(w, weight), np.float32).reshape(cfg.n_layers, d, n)
+        a[0, :, c] = 0.0
+        setattr(w, weight, a.ravel())
     else:
         cw = np.array(w.classifier_weights, np.float32)
         cw[d + c] = 7.0e4
@@ -297,6 +306,27 @@ def test_lm_head_input_beyond_limbs_in_prefill():
     report("prefill of 12 rows", rows, np.stack([rs.step(t, p) for p, t in enumerate(toks)]))
     for p in range(len(toks), len(toks) + 3):
         report(f"step {p}", dec.decode([0], [7], [p])[0], rs.step(7, p))
+    dec.close()
+    m.close()
+
+
+@pytest.mark.parametrize("where", ["ln1", "attention", "fc1"])
+def test_limb_overflow_in_prefill(where):
+    """A 12-row prefill whose first LayerNorm, attention or FC1 hands over f16 limbs of ~7e4: the rows run again in
+    full range and match the oracle, and so do the one-row steps and the nine rows after them, which read the keys
+    and values that the rerun wrote."""
+    cfg, w = overflow_model(where, 98)
+    m = ch.GpuModel(cfg, w, max_batch=1, max_len=16)
+    dec = ch.GpuDecoder(m, n_slots=1, max_len=32, max_rows=16)
+    rs = cr.RunState(cfg, w, max_len=32, num_threads=4)
+    toks = [0, 20, 5, 32, 11, 11, 23, 4, 17, 9, 30, 12]
+    rows = dec.decode(np.zeros(len(toks)), toks, np.arange(len(toks)))
+    report("prefill of 12 rows", rows, np.stack([rs.step(t, p) for p, t in enumerate(toks)]))
+    for p in range(len(toks), len(toks) + 2):
+        report(f"step {p}", dec.decode([0], [7], [p])[0], rs.step(7, p))
+    at = len(toks) + 2
+    rows = dec.decode(np.zeros(9), [4 + i for i in range(9)], at + np.arange(9))
+    report("nine more rows", rows, np.stack([rs.step(4 + i, at + i) for i in range(9)]))
     dec.close()
     m.close()
 

@@ -294,3 +294,50 @@ def test_plan_matches_the_routes_without_it(d, F, H, lens, dtype, monkeypatch):
     for k in ("logits", "hidden"):
         assert np.isfinite(got[0][k]).all()
         assert np.abs(got[0][k] - got[1][k]).max() <= 1e-5 * max(1.0, np.abs(got[1][k]).max()), k
+
+
+@pytest.mark.parametrize("d,F,H,lens", [
+    (640, 2560, 20, [49]), (640, 2560, 20, [63]),   # fewer rows than a 64-row tile
+    (640, 2560, 20, [390, 100]),                    # pair copies: FC1 on 64 x 128 tiles in two wave groups
+    (1280, 2560, 20, [257]),                        # QKV on those, also from the f16 copy
+    (1280, 5120, 20, [64]), (1280, 5120, 20, [200]), (1280, 5120, 20, [590])])  # FC1 in two, two and one group(s)
+@pytest.mark.parametrize("dtype", [0, 1])
+def test_plan_of_short_batches(d, F, H, lens, dtype, monkeypatch):
+    """49 to 600 rows, quantized and FP32 weights (pair copies), against the routes without the plan: 1e-5 of the
+    largest value, FP32 sums in another order."""
+    cfg = ch.EsmConfig(d, F, 1, H)
+    w = ch.EsmWeights.random(cfg, seed=d + 1, std=0.03, bias_std=0.02)
+    w = w.quantize_q8() if dtype == 1 else w
+    rng = np.random.default_rng(F)
+    seqs = [np.concatenate([[0], 4 + rng.integers(0, 20, n - 2), [2]]).astype(np.int32) for n in lens]
+    flags = ch.OUT_LOGITS | ch.OUT_HIDDEN
+    got = []
+    for env in (None, "0"):
+        if env:
+            monkeypatch.setenv("CIH_GEMM_PLAN", env)
+        m = ch.GpuModel(cfg, w, max_batch=len(seqs), max_len=max(lens), outputs=flags)
+        got.append(m.forward(seqs, flags))
+        m.close()
+    for k in ("logits", "hidden"):
+        assert np.isfinite(got[0][k]).all()
+        assert np.abs(got[0][k] - got[1][k]).max() <= 1e-5 * max(1.0, np.abs(got[1][k]).max()), k
+
+
+def test_split_320_tiles_of_a_partial_width(monkeypatch):
+    """128 x 320 tiles in k-splits with N = 480, whose second column tile is half empty (FC2, K = 2560, 6708 rows in two
+    splits): both block orders give the same bits, the routes without the plan the same to 1e-5 of the largest value."""
+    cfg = ch.EsmConfig(480, 2560, 1, 20)
+    w = ch.EsmWeights.random(cfg, seed=5, std=0.03, bias_std=0.02).quantize_q8()
+    rng = np.random.default_rng(5)
+    seqs = [np.concatenate([[0], 4 + rng.integers(0, 20, 514), [2]]).astype(np.int32) for _ in range(13)]
+    flags = ch.OUT_LOGITS | ch.OUT_HIDDEN
+    m = ch.GpuModel(cfg, w, max_batch=13, max_len=516, outputs=flags)
+    got = [m.forward(seqs, flags)]
+    for name in ("CIH_GEMM_SCHED", "CIH_GEMM_PLAN"):
+        with monkeypatch.context() as mp:
+            mp.setenv(name, "0")
+            got.append(m.forward(seqs, flags))
+    m.close()
+    for k in ("logits", "hidden"):
+        assert np.array_equal(got[0][k], got[1][k]), k
+        assert 0 < np.abs(got[0][k] - got[2][k]).max() <= 1e-5 * max(1.0, np.abs(got[2][k]).max()), k
