@@ -48,27 +48,38 @@ DTYPE_NOTE = ("GEMM activations as two f16 limbs (hi = f16(x), lo = f16(x - hi):
 # CIH_QGEMM=fp32 selects the FP32-MFMA kernel (1 MAC per MAC).
 
 
+def gemm_rows_on():
+    """Whether the few-rows GEMM is on: the switches that choose among the other GEMMs turn it off."""
+    env = os.environ.get
+    return (all(env(k) != "0" for k in ("CIH_GEMM_ROWS", "CIH_SPLITK", "CIH_GEMM_PLAN")) and
+            not any(k in os.environ for k in ("CIH_GEMM_LDS", "CIH_GEMM_TILE", "CIH_GEMM_TILE_N",
+                                              "CIH_GEMM_TILE_N_GELU", "CIH_GEMM_KW")))
+
+
 def qgemm_name(wname, T, d):
     """Which quantized GEMM the forward's projections take at T tokens: the
-    few-rows kernel from 9 to 48 tokens (to 64 for some projections), the
-    LDS-staged kernel above while the f16 copy of the quants is there, or, for a model loaded with CIH_GEMM_F16=0, when even the
-    narrowest projection (N = d) gives a full round of 128 x 128 tiles; else
-    the register-staged one (split-K for small T)."""
+    few-rows kernel from 9 to 48 tokens (for Wo and FC2 with K up to 5120 to
+    64), the LDS-staged kernel above while the f16 copy of the quants is there,
+    or, for a model loaded with CIH_GEMM_F16=0, when even the narrowest
+    projection (N = d) gives a full round of 128 x 128 tiles; else the
+    register-staged one (split-K for small T)."""
     env = os.environ.get
     copy = env("CIH_GEMM_F16") != "0"
+    rows = gemm_rows_on() and env("CIH_ACT") not in ("f32", "x3")
+    if rows and 8 < T <= 48:
+        return f"k_gemm_rows<{wname}> f16 MFMA, 2 limbs, W from the quants (QKV, Wo, FC1, FC2)"
     if env("CIH_GEMM_LDS") == "0":
         lds = False
     elif env("CIH_GEMM_LDS") == "force":
         lds = True
     elif copy and env("CIH_GEMM_PLAN") != "0":
-        if 8 < T <= 48 and env("CIH_GEMM_ROWS") != "0" and env("CIH_SPLITK") != "0":
-            return f"k_gemm_rows<{wname}> f16 MFMA, 2 limbs, W from the quants (QKV, Wo, FC1, FC2)"
         lds = T > 48
     else:
         lds = -(-T // 128) * -(-d // 128) >= 256
     if lds:
         src = "f16 copy of the quants" if copy else "quants"
-        return f"k_gemm_lds<{wname}> f16 MFMA, 2 limbs, operands global->LDS, W from the {src} (QKV, Wo, FC1, FC2)"
+        few = "QKV, FC1; k_gemm_rows: Wo, FC2 with K up to 5120" if rows and T <= 64 else "QKV, Wo, FC1, FC2"
+        return f"k_gemm_lds<{wname}> f16 MFMA, 2 limbs, operands global->LDS, W from the {src} ({few})"
     return f"k_gemm_x3<{wname}> f16 MFMA, 2 limbs (QKV, Wo, FC1, FC2)"
 
 
@@ -544,8 +555,11 @@ def main():
         elif fp32_model:
             # the f16 pair copy of the FP32 weights (hi and lo halves, K doubled)
             # times the activations' two f16 limbs: 4 f16 MFMA MACs per MAC
-            lds = T >= 64 and env("CIH_GEMM_LDS") != "0" and env("CIH_GEMM_PLAN") != "0" and env("CIH_ACT") != "f32"
-            kname = (("k_gemm_lds" if lds else "k_gemm_x3") + "<FP32 pair copy> f16 MFMA, 2 activation limbs x "
+            limbs_in = "CIH_ACT" not in os.environ
+            rows = limbs_in and T <= 48 and gemm_rows_on()
+            lds = limbs_in and T > 48 and "CIH_GEMM_LDS" not in os.environ and env("CIH_GEMM_PLAN") != "0"
+            kname = ("k_gemm_" + ("rows" if rows else "lds" if lds else "x3") +
+                     "<FP32 pair copy> f16 MFMA, 2 activation limbs x "
                      "2 weight halves (QKV, Wo, FC1, FC2, LM head)")
             peak, limbs = PEAK_F16_MFMA_TFLOPS, 4
         elif env("CIH_LIMBS") == "bf16x3":

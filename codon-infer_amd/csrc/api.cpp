@@ -443,8 +443,9 @@ int forward_impl(cih_model *m, const int32_t *tokens, const int32_t *lens, int32
     // f16-limb attention.
     // Other projections (GEMV, register-staged GEMMs, FP32 weights) write FP32
     // rows; from 2048 tokens on a prep kernel builds the same images from them,
-    // below that attention stages K/V itself (one launch less).  All paths
-    // give the same bits, so results do not depend on the batch they are in.
+    // below that attention stages K/V itself (one launch less).  These give
+    // the same bits; attention's splits over waves and key ranges, taken by
+    // batches that do not fill the device, regroup its sums.
     // CIH_ATT_IMG=prep: images by the prep kernel at any size.
     bool use_img = false, epi_img = false;
     int tile_rows = 0;

@@ -1686,11 +1686,13 @@ hipError_t launch_attention(const float *qkv, int d, int H, SeqMeta sm, const fl
     // the switches of the key split turn it off.
     const int nq32 = (sm.S_max + 31) / 32, t32 = sm.B * H * nq32;
     // Up to three tasks per CU it also pays on 4 waves, for sequences of at
-    // most 16 tiles and head sizes up to 32 (three workgroups fit a CU's LDS;
-    // no merge kernel) or with an export (no key split otherwise): 150M FP32
-    // B=3 (347, 61, 190) 2.76 -> 2.62 ms per forward, 150M Q8_0 B=3 2.49 -> 2.28,
-    // 8M FP32 B=3 with maps 0.405 -> 0.361, 650M Q8_0 B=2 (500, 300) with
-    // contacts 6.57 -> 6.37.  Not beyond: 35M B=4 (880 tasks) 0.804 -> 0.819,
+    // most 16 tiles and head sizes up to 32 (no merge kernel) or with an export
+    // (no key split otherwise).  By registers three workgroups share a CU at
+    // head size 16 and, without mixed heads, 32; two at 24, at 32 with mixed
+    // heads and at 64 with every head exported; one at 64 with mixed heads.
+    // 150M FP32 B=3 (347, 61, 190) 2.76 -> 2.62 ms per forward, 150M Q8_0 B=3
+    // 2.49 -> 2.28, 8M FP32 B=3 with maps 0.405 -> 0.361, with contacts 150M Q4_0
+    // B=3 2.66 -> 2.23, 650M Q8_0 B=2 (500, 300) 6.49 -> 6.19.  Not beyond: 35M B=4 (880 tasks) 0.804 -> 0.819,
     // 150M L=900 (29 tiles) 2.69 -> 2.74, 650M L=402 without an export 3.67 ->
     // 3.84.
     const bool split_on = !(se && !strcmp(se, "0")) && !(ke && !strcmp(ke, "0"));

@@ -1208,12 +1208,18 @@ int tile_choice(int M, int N, bool copy) {
 // Tile for an unsplit plain-epilogue GEMM from the f16 copy (or a pair copy:
 // 64-row tiles and 128 x 320 only) by the time its fullest CU takes: n tiles
 // of KB blocks, us, fitted to every tile measured on the ESM-2 35M to 3B
-// projections at 600 to 8192 rows (within 10% of them).  A CU's tiles share
+// projections at 600 to 8192 rows (within 10% of them; 64-row tiles on one
+// group of waves).  From 49 to 600 rows it differs from plain 64 x 64 tiles in
+// taking 64 x 128, on two groups where those fit one round: timed there, 2 to
+// 20% faster (650M QKV at 257 rows 16.4 -> 16.0 us, FC1 at 590 rows 32.5 ->
+// 28.5; 3B QKV at 200 rows 33.5 -> 28.4, FC1 at 320 rows 60 -> 51.5) but for the
+// pair copy of 150M FC1 at 385 to 600 rows (16.8 -> 17.3).  A CU's tiles share
 // its matrix cores, so the 64-row tiles' times add up; 128 x 128 tiles run in
 // pairs; the 8-wave tiles one after the other (128 x 320 over several rounds
-// with plain epilogues as persistent workgroups).  What it corrects: FC1 of
-// 35M at 2729 rows 24.6 -> 20.3 us (64 x 128 instead of 128 x 256), of 150M
-// at 2100 rows 27.4 -> 24.2, of 650M at 700 rows 33.6 -> 29.6.
+// with plain epilogues as persistent workgroups).  Against the round model
+// and 64 x 64 tiles: FC1 of 35M at 2729 rows 26.4 -> 22.5 us (64 x 128 instead
+// of 128 x 256), of 150M at 2100 rows 29.8 -> 26.5, of 650M at 700 rows 36.5 ->
+// 31.6.
 int tile_time(int M, int N, int KB, bool pair, int epi) {
     const long cus = device_cus(), m64 = (M + 63) / 64, m128 = (M + 127) / 128;
     auto fullest = [&](long mt, int bn) { return (double)((mt * ((N + bn - 1) / bn) + cus - 1) / cus); };

@@ -22,16 +22,18 @@
 //     about 45 B/ns from L2, so CT and the split are chosen for the fewest
 //     bytes per CU (rows_plan).
 //
-// Against the register-staged GEMM with its split-K reductions (us per
-// launch, weights cold, the LayerNorm that adds the splits included): 650M
-// Q8_0 at 41 rows QKV 12.7 -> 9.9, Wo 9.9 -> 9.1, FC1 14.6 -> 10.9, FC2 16.0
-// -> 11.7; at 9 rows 10.1 -> 4.6, 9.0 -> 7.7, 11.0 -> 6.3, 13.0 -> 8.7.
-// Floors at 41 rows: 1.2 us for QKV's 5.5 MB at the 4.8 TB/s of a large copy,
-// about 2.5 us for the launch.  One 41-token sequence of 650M Q8_0: 2.33 ->
-// 2.00 ms per forward.  Tried: activations staged in LDS for 64-column
-// workgroups with K split over the device and a fold kernel (QKV 10.9 us at
-// 41 rows: the fold's 4.6 us eats the gain), 8 rows x 2 limbs per MFMA
-// (10.1), workgroups starting at different k-blocks (no change).
+// Against the register-staged GEMM, traced inside a 650M Q8_0 forward (us;
+// before: QKV and FC1 with the reduction kernel of their splits; the LayerNorm
+// that adds Wo's and FC2's is apart, 5.8 -> 4.9): at 41 rows QKV 13.7 -> 12.5,
+// Wo 6.1 -> 5.1, FC1 15.8 -> 13.4, FC2 10.6 -> 7.6; at 9 rows 11.6 -> 5.4, 5.4
+// -> 4.8, 12.2 -> 8.1, 7.7 -> 4.8.  Timed alone, with their activations read
+// before, QKV and FC1 of 41 rows take 9.9 and 10.9.  Floors at 41 rows: 1.2 us
+// for QKV's 5.5 MB at the 4.8 TB/s of a large copy, about 2.5 us for the
+// launch.  One 41-token sequence of 650M Q8_0: 2.33 -> 2.00 ms per forward.
+// Tried, alone: activations staged in LDS for 64-column workgroups with K
+// split over the device and a fold kernel (QKV 10.9 us at 41 rows: the fold's
+// 4.6 us eats the gain), 8 rows x 2 limbs per MFMA (10.1), workgroups starting
+// at different k-blocks (no change).
 #include <stdlib.h>
 #include <string.h>
 
@@ -199,7 +201,7 @@ bool gemm_rows_applies(const DevMatrix &W, int a_fmt, int M, int epi) {
     if (epi == EPI_GELU_H2 && W.N % 32) return false;
     // From 49 rows on the LDS GEMM's 64-row tiles take over, except where K is
     // short or the LayerNorm after the projection adds many splits anyway
-    // (us at 48 / 64 rows, this kernel against 64 x 64 tiles: 650M QKV 10.5 /
+    // (timed alone, us at 48 / 64 rows, this kernel against 64 x 64 tiles: 650M QKV 10.5 /
     // 12.5 against 10.6 / 10.7, FC1 11.5 / 13.5 against 12.6 / 12.7, FC2 with
     // its LayerNorm 12.0 / 13.6 against 14.7 / 15.0; 35M QKV 5.3 / 6.1 against
     // 6.0 / 5.7; 8M FC1 4.4 / 5.0 against 5.8 / 5.4; 3B FC2 21.8 / 28.6 against
@@ -246,8 +248,9 @@ static hipError_t launch_rows_w(const DevMatrix &W, int KB, int KBX, const unsig
 // workgroups' activations and weights, one after the other when there are
 // more than CUs), at the 45 B/ns a CU gets from L2.  Splits add the partial
 // sums' traffic (4 TB/s) and, unless the caller folds them into its next
-// kernel, a fold launch of 4.6 us.  Within 5% of the best of CT x S measured
-// on the ESM-2 projections at 9 to 48 rows.
+// kernel, a fold launch of 4.6 us.  Within 5% of the best of CT x S timed alone
+// on the ESM-2 projections at 9 to 48 rows; inside a forward, where the wide
+// projections take 1 to 3 us more, the choices have not been compared.
 static void rows_plan(int M, int N, int KB, bool deferred, size_t part_floats, double wbyte, int &ct, int &S) {
     const long cus = device_cus();
     const double rowb = (M + 15) / 16 * 16 * 128.0;
