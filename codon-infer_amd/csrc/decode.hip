@@ -5,6 +5,8 @@
 // (codon-infer src/lib.rs:3616-3663, 3438-3483).
 #include <math.h>
 
+#include <type_traits>
+
 #include "head_wo.h"
 #include "kernels.h"
 #include "x3.h"
@@ -73,8 +75,8 @@ __device__ __forceinline__ float block_reduce(float v, float *scratch, bool is_m
 // 1 / sum), then out = sum_t p_t v_t.  Bound by reading the slot's K and V
 // (512 bytes a key at hd 64) at the 45 B/ns a CU takes: L = HD / 4 lanes read
 // a row in 16-byte pieces, so a wave's load covers 64 / L whole rows, and
-// each wave has U such loads in flight, the first U of K and of V requested
-// before anything else.  A key's score is added over its lanes, an output
+// each wave has U such loads in flight (eight, or 1, 2 or 4 that cover all
+// keys), the first U of K and of V requested before anything else.  A key's score is added over its lanes, an output
 // dim over a lane's keys, the wave's key groups and the waves, in that order.
 // (A thread per key row, and V rows four at a time by 64 lanes, took 28.8 us
 // per layer for 8 rows at position 700 of 650M and 13.9 us for one at 280;
@@ -108,8 +110,7 @@ __global__ __launch_bounds__(ATT_THREADS) void k_decode_attention(const float *_
                                                                   int wo_n = 0) {
     constexpr int HALF = HD / 2, NWV = ATT_THREADS / 64;
     constexpr int LK = HD == 24 ? 8 : HD / 4;  // lanes per key (hd 24: lanes 6 and 7 of 8 idle)
-    constexpr int KW = 64 / LK, U = 8;         // keys per load of a wave, loads in flight
-    constexpr int STEP = NWV * KW * U;         // keys per sweep of the workgroup
+    constexpr int KW = 64 / LK;                // keys per load of a wave
     extern __shared__ __attribute__((aligned(16))) float sm[];
     float *qs = sm;                        // [HD] rotated query
     float *kcur = qs + HD, *vcur = kcur + HD;  // [HD] key and value at pos (FUSED)
@@ -133,122 +134,134 @@ __global__ __launch_bounds__(ATT_THREADS) void k_decode_attention(const float *_
     const bool live = lane % LK < HD / 4;
     const float *Kl = K + dl, *Vl = V + dl;
     auto key = [&](int s0, int u) __attribute__((always_inline)) { return s0 + (u * NWV + wave) * KW + kq; };
-    // keys past the cached ones re-read the last (their scores are not stored, their weights zero)
-    auto fetch = [&](const float *base, int s0, f32x4 (&v)[U]) __attribute__((always_inline)) {
+    f32x4 o4 = {0.0f, 0.0f, 0.0f, 0.0f};
+    auto attend = [&](auto UU) __attribute__((always_inline)) {
+        // keys past the cached ones re-read the last (their scores are not stored, their weights zero)
+        constexpr int U = decltype(UU)::value, STEP = NWV * KW * U;  // loads in flight, keys per sweep of the workgroup
+        auto fetch = [&](const float *base, int s0, f32x4 (&v)[U]) __attribute__((always_inline)) {
 #pragma unroll
-        for (int u = 0; u < U; u++)
-            v[u] = *reinterpret_cast<const f32x4 *>(base + (size_t)min(key(s0, u), n_cached - 1) * d);
-    };
-    // The first sweep of K and of V is requested before anything waits, so its
-    // latency overlaps the gather, the rotation, the softmax and the barriers.
-    f32x4 kv[U], vv[U];
-    if (n_cached > 0) {
-        fetch(Kl, 0, kv);
-        fetch(Vl, 0, vv);
-    }
-    if constexpr (FUSED) {
-        float c = 0.0f, s = 0.0f;
-        if (t < HALF) {
-            c = rc[(size_t)pos * HALF + t];
-            s = rs[(size_t)pos * HALF + t];
+            for (int u = 0; u < U; u++)
+                v[u] = *reinterpret_cast<const f32x4 *>(base + (size_t)min(key(s0, u), n_cached - 1) * d);
+        };
+        // The first sweep of K and of V is requested before anything waits, so its
+        // latency overlaps the gather, the rotation, the softmax and the barriers.
+        f32x4 kv[U], vv[U];
+        if (n_cached > 0) {
+            fetch(Kl, 0, kv);
+            fetch(Vl, 0, vv);
         }
-        // this head's q, k, v: the row of qkv, or the GEMV's partial sums
-        // (eight interleaved sums over the splits) + bias
-        if (t < 3 * HD) {
-            const int which = t / HD, col = which * d + h * HD + (t - which * HD);
-            float v;
-            if (part) {
-                const size_t stride = (size_t)gridDim.x * 3 * d;
-                const float *pp = part + (size_t)r * 3 * d + col;
-                float a[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
-                int y = 0;
-                for (; y + 8 <= splits; y += 8) {
-#pragma unroll
-                    for (int u = 0; u < 8; u++) a[u] += pp[(y + u) * stride];
-                }
-                for (int u = 0; y < splits; y++, u++) a[u] += pp[y * stride];
-                v = (((a[0] + a[1]) + (a[2] + a[3])) + ((a[4] + a[5]) + (a[6] + a[7]))) + bias[col];
-            } else {
-                v = qkv[(size_t)r * 3 * d + col];
+        if constexpr (FUSED) {
+            float c = 0.0f, s = 0.0f;
+            if (t < HALF) {
+                c = rc[(size_t)pos * HALF + t];
+                s = rs[(size_t)pos * HALF + t];
             }
-            qs[t] = v;  // qs | kcur | vcur are contiguous
+            // this head's q, k, v: the row of qkv, or the GEMV's partial sums
+            // (eight interleaved sums over the splits) + bias
+            if (t < 3 * HD) {
+                const int which = t / HD, col = which * d + h * HD + (t - which * HD);
+                float v;
+                if (part) {
+                    const size_t stride = (size_t)gridDim.x * 3 * d;
+                    const float *pp = part + (size_t)r * 3 * d + col;
+                    float a[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+                    int y = 0;
+                    for (; y + 8 <= splits; y += 8) {
+#pragma unroll
+                        for (int u = 0; u < 8; u++) a[u] += pp[(y + u) * stride];
+                    }
+                    for (int u = 0; y < splits; y++, u++) a[u] += pp[y * stride];
+                    v = (((a[0] + a[1]) + (a[2] + a[3])) + ((a[4] + a[5]) + (a[6] + a[7]))) + bias[col];
+                } else {
+                    v = qkv[(size_t)r * 3 * d + col];
+                }
+                qs[t] = v;  // qs | kcur | vcur are contiguous
+            }
+            __syncthreads();
+            // apply_rope (lib.rs:3533-3552) for this head, products rounded one by one
+            if (t < HALF) {
+                const float q0 = qs[t], q1 = qs[t + HALF], k0 = kcur[t], k1 = kcur[t + HALF];
+                qs[t] = __fsub_rn(__fmul_rn(q0, c), __fmul_rn(q1, s));
+                qs[t + HALF] = __fadd_rn(__fmul_rn(q1, c), __fmul_rn(q0, s));
+                const float r0 = __fsub_rn(__fmul_rn(k0, c), __fmul_rn(k1, s));
+                const float r1 = __fadd_rn(__fmul_rn(k1, c), __fmul_rn(k0, s));
+                kcur[t] = r0;
+                kcur[t + HALF] = r1;
+                if (cache_writer) {
+                    K[(size_t)pos * d + t] = r0;
+                    K[(size_t)pos * d + t + HALF] = r1;
+                }
+            } else if (t >= 64 && t < 64 + HD && cache_writer) {
+                V[(size_t)pos * d + t - 64] = vcur[t - 64];
+            }
+        } else {
+            const float *q = qkv + (size_t)r * 3 * d + h * HD;
+            if (t < HD) qs[t] = q[t];
         }
         __syncthreads();
-        // apply_rope (lib.rs:3533-3552) for this head, products rounded one by one
-        if (t < HALF) {
-            const float q0 = qs[t], q1 = qs[t + HALF], k0 = kcur[t], k1 = kcur[t + HALF];
-            qs[t] = __fsub_rn(__fmul_rn(q0, c), __fmul_rn(q1, s));
-            qs[t + HALF] = __fadd_rn(__fmul_rn(q1, c), __fmul_rn(q0, s));
-            const float r0 = __fsub_rn(__fmul_rn(k0, c), __fmul_rn(k1, s));
-            const float r1 = __fadd_rn(__fmul_rn(k1, c), __fmul_rn(k0, s));
-            kcur[t] = r0;
-            kcur[t + HALF] = r1;
-            if (cache_writer) {
-                K[(size_t)pos * d + t] = r0;
-                K[(size_t)pos * d + t + HALF] = r1;
+        const f32x4 q4 = *reinterpret_cast<const f32x4 *>(qs + dl);
+        // a key's products over its lanes: DPP adds within 16 lanes (quads, halves
+        // of 8, mirrored: partners hold equal sums by then)
+        auto key_sum = [&](f32x4 k) __attribute__((always_inline)) {
+            float a = live ? fmaf(q4.w, k.w, fmaf(q4.z, k.z, fmaf(q4.y, k.y, q4.x * k.x))) : 0.0f;
+            a += dpp<0xB1>(a);                            // lane ^ 1
+            a += dpp<0x4E>(a);                            // lane ^ 2
+            if constexpr (LK >= 8) a += dpp<0x141>(a);    // mirrored in 8
+            if constexpr (LK >= 16) a += dpp<0x140>(a);   // mirrored in 16
+            return a;
+        };
+        for (int s0 = 0; s0 < n_cached; s0 += STEP) {
+            float a[U];
+#pragma unroll
+            for (int u = 0; u < U; u++) a[u] = key_sum(kv[u]);
+            if (s0 + STEP < n_cached) fetch(Kl, s0 + STEP, kv);
+#pragma unroll
+            for (int u = 0; u < U; u++)
+                if (lane % LK == 0 && key(s0, u) < n_cached) p[key(s0, u)] = a[u] * inv_scale;
+        }
+        if (FUSED && wave == 0) {
+            const float a = key_sum(*reinterpret_cast<const f32x4 *>(kcur + dl));
+            if (lane == 0) p[pos] = a * inv_scale;
+        }
+        __syncthreads();
+        float mx = -INFINITY;
+        for (int j = t; j <= pos; j += ATT_THREADS) mx = fmaxf(mx, p[j]);
+        mx = block_reduce(mx, red, true);
+        float sum = 0.0f;
+        for (int j = t; j <= pos; j += ATT_THREADS) {
+            const float e = expf(p[j] - mx);
+            p[j] = e;
+            sum += e;
+        }
+        sum = block_reduce(sum, red, false);
+        const float inv = 1.0f / sum;
+        __syncthreads();
+        for (int s0 = 0; s0 < n_cached; s0 += STEP) {
+            if (s0 > 0) fetch(Vl, s0, vv);
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                const int j = key(s0, u);
+                const float w = j < n_cached ? p[j] * inv : 0.0f;
+#pragma unroll
+                for (int e = 0; e < 4; e++) o4[e] = fmaf(w, vv[u][e], o4[e]);
             }
-        } else if (t >= 64 && t < 64 + HD && cache_writer) {
-            V[(size_t)pos * d + t - 64] = vcur[t - 64];
         }
-    } else {
-        const float *q = qkv + (size_t)r * 3 * d + h * HD;
-        if (t < HD) qs[t] = q[t];
-    }
-    __syncthreads();
-    const f32x4 q4 = *reinterpret_cast<const f32x4 *>(qs + dl);
-    // a key's products over its lanes: DPP adds within 16 lanes (quads, halves
-    // of 8, mirrored: partners hold equal sums by then)
-    auto key_sum = [&](f32x4 k) __attribute__((always_inline)) {
-        float a = live ? fmaf(q4.w, k.w, fmaf(q4.z, k.z, fmaf(q4.y, k.y, q4.x * k.x))) : 0.0f;
-        a += dpp<0xB1>(a);                            // lane ^ 1
-        a += dpp<0x4E>(a);                            // lane ^ 2
-        if constexpr (LK >= 8) a += dpp<0x141>(a);    // mirrored in 8
-        if constexpr (LK >= 16) a += dpp<0x140>(a);   // mirrored in 16
-        return a;
+        if (FUSED && wave == 0 && kq == 0) {
+            const float w = p[pos] * inv;
+            const f32x4 v = *reinterpret_cast<const f32x4 *>(vcur + dl);
+#pragma unroll
+            for (int e = 0; e < 4; e++) o4[e] = fmaf(w, v[e], o4[e]);
+        }
     };
-    for (int s0 = 0; s0 < n_cached; s0 += STEP) {
-        float a[U];
-#pragma unroll
-        for (int u = 0; u < U; u++) a[u] = key_sum(kv[u]);
-        if (s0 + STEP < n_cached) fetch(Kl, s0 + STEP, kv);
-#pragma unroll
-        for (int u = 0; u < U; u++)
-            if (lane % LK == 0 && key(s0, u) < n_cached) p[key(s0, u)] = a[u] * inv_scale;
-    }
-    if (FUSED && wave == 0) {
-        const float a = key_sum(*reinterpret_cast<const f32x4 *>(kcur + dl));
-        if (lane == 0) p[pos] = a * inv_scale;
-    }
-    __syncthreads();
-    float mx = -INFINITY;
-    for (int j = t; j <= pos; j += ATT_THREADS) mx = fmaxf(mx, p[j]);
-    mx = block_reduce(mx, red, true);
-    float sum = 0.0f;
-    for (int j = t; j <= pos; j += ATT_THREADS) {
-        const float e = expf(p[j] - mx);
-        p[j] = e;
-        sum += e;
-    }
-    sum = block_reduce(sum, red, false);
-    const float inv = 1.0f / sum;
-    __syncthreads();
-    f32x4 o4 = {0.0f, 0.0f, 0.0f, 0.0f};
-    for (int s0 = 0; s0 < n_cached; s0 += STEP) {
-        if (s0 > 0) fetch(Vl, s0, vv);
-#pragma unroll
-        for (int u = 0; u < U; u++) {
-            const int j = key(s0, u);
-            const float w = j < n_cached ? p[j] * inv : 0.0f;
-#pragma unroll
-            for (int e = 0; e < 4; e++) o4[e] = fmaf(w, vv[u][e], o4[e]);
-        }
-    }
-    if (FUSED && wave == 0 && kq == 0) {
-        const float w = p[pos] * inv;
-        const f32x4 v = *reinterpret_cast<const f32x4 *>(vcur + dl);
-#pragma unroll
-        for (int e = 0; e < 4; e++) o4[e] = fmaf(w, v[e], o4[e]);
-    }
+    // As many loads in flight as the cached keys fill, up to eight: the ones past
+    // the last key would still pass through the CU's load path (with eight
+    // throughout: 8M Q4_0, a prompt of 439 rows 0.73 -> 0.62 ms; 650M Q4_0, one
+    // stream at position 30 1.038 -> 0.989 ms per step)
+    const int need = (n_cached + NWV * KW - 1) / (NWV * KW);
+    if (need <= 1) attend(std::integral_constant<int, 1>{});
+    else if (need <= 2) attend(std::integral_constant<int, 2>{});
+    else if (need <= 4) attend(std::integral_constant<int, 4>{});
+    else attend(std::integral_constant<int, 8>{});
     // the wave's key groups, then the waves
 #pragma unroll
     for (int o = LK; o < 64; o <<= 1)

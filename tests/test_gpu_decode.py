@@ -335,8 +335,8 @@ def test_limb_overflow_in_prefill(where):
 @pytest.mark.parametrize("hd,rows", [(64, 530), (32, 530), (24, 530), (16, 1040)])
 def test_decode_attention_past_one_sweep(hd, rows):
     """Keys past the attention workgroup's one (256 at hd 64, 512 at 32 and 24, 1024 at 16) and two sweeps: a prompt
-    prefilled in one call, then single steps at the edges of the sweeps (which rewrite those positions), against the
-    oracle's one-token forwards."""
+    prefilled in one call, then single steps at the edges of the sweeps and of their loads (which rewrite those
+    positions), against the oracle's one-token forwards."""
     cfg = ch.EsmConfig(2 * hd if hd != 24 else 96, 128, 2, 2 if hd != 24 else 4, max_seq_len=rows)
     w = ch.EsmWeights.random(cfg, seed=hd, std=0.08, bias_std=0.02).quantize_q8()
     rng = np.random.default_rng(hd)
@@ -348,7 +348,8 @@ def test_decode_attention_past_one_sweep(hd, rows):
     ref = np.stack([rs.step(int(t), p) for p, t in enumerate(toks)])
     assert np.abs(got - ref).max() <= 1e-3
     step = {64: 256, 32: 512, 24: 512, 16: 1024}[hd]
-    for p in sorted({1, 2, step - 1, step, step + 1, rows - 1} | ({2 * step, 2 * step + 1} if 2 * step + 1 < rows else set())):
+    loads = {e + i * step // 8 for i in (1, 2, 4) for e in (-1, 0, 1)}  # 1, 2 and 4 of a sweep's eight loads
+    for p in sorted(loads | {1, 2, step - 1, step, step + 1, rows - 1} | ({2 * step, 2 * step + 1} if 2 * step + 1 < rows else set())):
         one = dec.decode([0], [toks[p]], [p])[0]
         assert np.abs(one - ref[p]).max() <= 1e-3, p
     dec.close()
